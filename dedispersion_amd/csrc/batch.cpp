@@ -156,13 +156,15 @@ template <typename L> void merge_geometry(KindQueue &k, const L &launch, bool fi
     k.g.lds_bytes = std::max(k.g.lds_bytes, launch.g.lds_bytes);
     k.g.win = std::max(k.g.win, launch.g.win);
     k.g.packed |= launch.g.packed;
+    k.g.wide |= launch.g.wide;
   }
 }
 
 // Every job's launches under the batch configuration (and its plan's own),
 // sorted into the kind queues or beside them; `pairs`: prepare the compact
-// step two's paired kernel where a job allows it.
-dd_status plan_jobs(dd_batch *b, bool pairs) {
+// step two's paired kernel where a job allows it; `single`, `one`: the form
+// of the byte kernel of the single-step and step-one jobs.
+dd_status plan_jobs(dd_batch *b, bool pairs, ByteKernel single, ByteKernel one) {
   for (auto &k : b->q) {
     k.u8.clear();
     k.f32.clear();
@@ -191,7 +193,8 @@ dd_status plan_jobs(dd_batch *b, bool pairs) {
       s = prepare_single(job.plan, job.plan->conf[DD_SINGLE_STEP], job.in, job.out, job.first_sbeam, job.nr_sbeams,
                          P);
       if (s != DD_OK) return s;
-      s = prepare_single(job.plan, b->conf[DD_SINGLE_STEP], job.in, job.out, job.first_sbeam, job.nr_sbeams, L);
+      s = prepare_single(job.plan, b->conf[DD_SINGLE_STEP], job.in, job.out, job.first_sbeam, job.nr_sbeams, L,
+                         single);
       if (s != DD_OK && s != DD_ERR_CONFIGURATION) return s;
       b->pj_single.push_back(P);
       b->units += sbeams * o.nr_dms * z.nr_samples;
@@ -219,7 +222,7 @@ dd_status plan_jobs(dd_batch *b, bool pairs) {
       b->units += sbeams * o.nr_dms_subbanding * o.nr_dms * z.nr_samples;
       U8Launch L1;
       F32Launch L2;
-      s = prepare_step_one(job.plan, b->conf[DD_STEP_ONE], job.in, job.mid, L1);
+      s = prepare_step_one(job.plan, b->conf[DD_STEP_ONE], job.in, job.mid, L1, one);
       if (s == DD_OK)
         s = prepare_step_two(job.plan, b->conf[DD_STEP_TWO], job.mid, job.out, job.first_sbeam, job.nr_sbeams, L2);
       // the plan's own launches prepared above; a batch configuration that
@@ -257,6 +260,15 @@ dd_status plan_jobs(dd_batch *b, bool pairs) {
   return DD_OK;
 }
 
+// One kernel runs all jobs of a kind: where the plans' rules differ, the form
+// that holds most of the tiles (kByRule: they agree).
+ByteKernel common_byte_kernel(const KindQueue &k) {
+  uint64_t tiles[2] = {0, 0};
+  for (const U8Launch &L : k.u8) tiles[L.g.matrix ? 1 : 0] += L.k.n_tiles;
+  if (tiles[0] == 0 || tiles[1] == 0) return ByteKernel::kByRule;
+  return tiles[1] >= tiles[0] ? ByteKernel::kMatrix : ByteKernel::kVector;
+}
+
 // The host part of build(): every job's launches, the per-kind geometry,
 // occupancy and tile lists (tiles[m] for kind m); no device memory is
 // touched.
@@ -285,16 +297,24 @@ dd_status plan_batch(dd_batch *b, std::vector<TileDesc> (&tiles_of)[3]) {
     if (job.kind == kTwoStep && 255u * std::max(job.plan->max_live_sub, 1u) > 65535u) b->compact = false;
   // one step-two kernel for the whole batch: the paired one only when every
   // job in the batch kernels took it
-  bool pairs = b->compact && b->paired_requested;
-  dd_status st = plan_jobs(b, pairs);
+  const bool pairs = b->compact && b->paired_requested;
+  dd_status st = plan_jobs(b, pairs, ByteKernel::kByRule, ByteKernel::kByRule);
   if (st != DD_OK) return st;
-  if (pairs) {
-    bool all = true;
-    for (const F32Launch &L : b->q[DD_STEP_TWO].f32) all = all && L.g.pairs;
-    if (!all) {
-      st = plan_jobs(b, false);
-      if (st != DD_OK) return st;
-    }
+  bool all = true;
+  for (const F32Launch &L : b->q[DD_STEP_TWO].f32) all = all && L.g.pairs;
+  ByteKernel single = common_byte_kernel(b->q[DD_SINGLE_STEP]), one = common_byte_kernel(b->q[DD_STEP_ONE]);
+  if ((pairs && !all) || single != ByteKernel::kByRule || one != ByteKernel::kByRule) {
+    st = plan_jobs(b, pairs && all, single, one);
+    if (st != DD_OK) return st;
+  }
+  // a job that the matrix form has no room for (its row window) takes the others with it
+  const bool mixed_single = common_byte_kernel(b->q[DD_SINGLE_STEP]) != ByteKernel::kByRule;
+  const bool mixed_one = common_byte_kernel(b->q[DD_STEP_ONE]) != ByteKernel::kByRule;
+  if (mixed_single || mixed_one) {
+    if (mixed_single) single = ByteKernel::kVector;
+    if (mixed_one) one = ByteKernel::kVector;
+    st = plan_jobs(b, pairs && all, single, one);
+    if (st != DD_OK) return st;
   }
   for (int m = 0; m < 3; ++m) {
     KindQueue &k = b->q[m];

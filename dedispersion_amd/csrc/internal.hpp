@@ -147,6 +147,8 @@ struct Geometry {
   uint32_t packed;     // 1 = the rows may be packed (RowSumU8Params::in_log2f)
   uint32_t unroll;     // rows staged per barrier (the configuration's, or its cap)
   uint32_t pairs;      // 1 = the paired uint16 step two (kernels_u16_pairs.hip)
+  uint32_t matrix;     // 1 = the matrix-core form of the staged kernel (kernels_u8_matrix.hip)
+  uint32_t wide;       // 1 = ... whose rows may take more than one window
 };
 
 // Launchers (kernels_u8.hip / kernels_f32.hip).  Return hipSuccess or the
@@ -215,6 +217,16 @@ hipError_t launch_rowsum_u16_pairs_list(const RowSumF32Params *d_jobs, const Til
                                         const Geometry &g, hipStream_t stream);
 hipError_t rowsum_u16_pairs_batch_occupancy(const Geometry &g, int *per_cu);
 inline uint32_t u16_staged_chunks(uint32_t run) { return run / 8 + 1; }  // 16-byte loads per lane per row
+// The matrix-core form of the staged byte kernels (kernels_u8_matrix.hip;
+// Geometry::matrix, items_d1 4 or 8).
+hipError_t launch_rowsum_u8_matrix(const RowSumU8Params &p, const Geometry &g, hipStream_t stream);
+hipError_t launch_rowsum_u8_matrix_batch(const RowSumU8Params *d_jobs, const TileQueues &q, const Geometry &g,
+                                         uint32_t workgroups, hipStream_t stream);
+hipError_t launch_rowsum_u8_matrix_list(const RowSumU8Params *d_jobs, const TileDesc *d_tiles, uint32_t n,
+                                        const Geometry &g, hipStream_t stream);
+hipError_t rowsum_u8_matrix_batch_occupancy(const Geometry &g, int *per_cu);
+constexpr uint32_t kU8MatrixReach = 32;     // bytes that its operands reach past a row's window
+constexpr uint32_t kU8MatrixWindow = 2048;  // widest row window that it stages (two loads per wavefront)
 constexpr uint32_t kStagedSlotsPerWave = 2;  // rows staged per wavefront per group
 constexpr uint32_t kU8StagedChunks = 2;      // 16-byte staging loads per lane per row (window <= 2 KiB)
 inline uint32_t f32_staged_chunks(uint32_t run) { return run / 4 + 1; }

@@ -30,61 +30,12 @@
 // a time (lane l: DM 2s + l / 32 of the wavefront's DMs, over the groups
 // (l % 32) + 32q), so every lane reads its own DM's LDS address.
 #include "staged_common.hpp"
+#include "u8_unpack.hpp"
 
 namespace ddamd {
 namespace {
 
 using namespace staged;
-
-// The 16 samples of window group m (one byte each, 4 dwords u) and the 4
-// after them (`next`) from the packed dwords d[0..2], which start at the
-// dword holding packed byte 16m >> LF; LF = log2 of samples per byte (1..3).
-// Samples are the fields of each byte from the least significant bit up.
-template <int LF>
-__device__ __forceinline__ void unpack_group(const u32x4 &d, uint32_t m, uint32_t (&u)[4], uint32_t &next) {
-  if constexpr (LF == 1) {
-    // 4-bit fields, 64 bits from d[0] and d[1] (the next 4 samples in the low
-    // half of d[2]): even fields to the bytes of `lo`, odd fields to those
-    // of `hi`, interleaved
-#pragma unroll
-    for (int e = 0; e < 3; ++e) {
-      const uint32_t lo = d[e] & 0x0F0F0F0Fu, hi = (d[e] >> 4) & 0x0F0F0F0Fu;
-      const uint32_t a = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
-      if (e < 2) {
-        u[2 * e] = a;
-        u[2 * e + 1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
-      } else {
-        next = a;
-      }
-    }
-  } else if constexpr (LF == 2) {
-    // 2-bit fields, 32 bits from d[0] (the next 4 samples in the low byte of
-    // d[1]): m_j byte k = sample 4k + j; two rounds of byte interleave
-    const uint32_t x = d[0];
-    const uint32_t m0 = x & 0x03030303u, m1 = (x >> 2) & 0x03030303u;
-    const uint32_t m2 = (x >> 4) & 0x03030303u, m3 = (x >> 6) & 0x03030303u;
-    const uint32_t a01 = __builtin_amdgcn_perm(m1, m0, 0x05010400u);  // s0 s1 s4 s5
-    const uint32_t a23 = __builtin_amdgcn_perm(m3, m2, 0x05010400u);  // s2 s3 s6 s7
-    const uint32_t b01 = __builtin_amdgcn_perm(m1, m0, 0x07030602u);  // s8 s9 s12 s13
-    const uint32_t b23 = __builtin_amdgcn_perm(m3, m2, 0x07030602u);  // s10 s11 s14 s15
-    u[0] = __builtin_amdgcn_perm(a23, a01, 0x05040100u);
-    u[1] = __builtin_amdgcn_perm(a23, a01, 0x07060302u);
-    u[2] = __builtin_amdgcn_perm(b23, b01, 0x05040100u);
-    u[3] = __builtin_amdgcn_perm(b23, b01, 0x07060302u);
-    const uint32_t y = d[1];
-    const uint32_t c01 = __builtin_amdgcn_perm((y >> 2) & 0x03030303u, y & 0x03030303u, 0x05010400u);
-    const uint32_t c23 = __builtin_amdgcn_perm((y >> 6) & 0x03030303u, (y >> 4) & 0x03030303u, 0x05010400u);
-    next = __builtin_amdgcn_perm(c23, c01, 0x05040100u);
-  } else {
-    // 1-bit fields, 16 bits from bit 16 (m & 1) of d[0]: a nibble n spread to
-    // bytes by n * (1 + 2^7 + 2^14 + 2^21), whose four shifted copies do not
-    // overlap, then bit 0 of each byte kept
-    const uint32_t x = __builtin_amdgcn_alignbit(d[1], d[0], 16 * (m & 1));
-#pragma unroll
-    for (int q = 0; q < 4; ++q) u[q] = (((x >> (4 * q)) & 0xFu) * 0x204081u) & 0x01010101u;
-    next = (((x >> 16) & 0xFu) * 0x204081u) & 0x01010101u;
-  }
-}
 
 // Writes the byte run u (n dwords, followed by the dword `next`) to the
 // four copies of a row window at dword position `at`: copy c holds the run
@@ -524,6 +475,7 @@ template <typename F> hipError_t dispatch(const Geometry &g, bool flush, F &&f) 
 } // namespace
 
 hipError_t launch_rowsum_u8_staged(const RowSumU8Params &p, const Geometry &g, bool flush, hipStream_t stream) {
+  if (g.matrix) return launch_rowsum_u8_matrix(p, g, stream);
   return dispatch(g, flush, [&](auto run, auto dpw, auto fl, auto pk) {
     hipLaunchKernelGGL((rowsum_u8_staged<run.value, dpw.value, fl.value, pk.value>), dim3(p.n_tiles), dim3(64 * g.threads_d1),
                        g.lds_bytes, stream, p);
@@ -533,6 +485,7 @@ hipError_t launch_rowsum_u8_staged(const RowSumU8Params &p, const Geometry &g, b
 
 hipError_t launch_rowsum_u8_batch(const RowSumU8Params *d_jobs, const TileQueues &q, const Geometry &g, bool flush,
                                   uint32_t workgroups, hipStream_t stream) {
+  if (g.matrix) return launch_rowsum_u8_matrix_batch(d_jobs, q, g, workgroups, stream);
   return dispatch(g, flush, [&](auto run, auto dpw, auto fl, auto pk) {
     hipLaunchKernelGGL((rowsum_u8_batch<run.value, dpw.value, fl.value, pk.value>), dim3(workgroups), dim3(64 * g.threads_d1),
                        g.lds_bytes, stream, d_jobs, q);
@@ -542,6 +495,7 @@ hipError_t launch_rowsum_u8_batch(const RowSumU8Params *d_jobs, const TileQueues
 
 hipError_t launch_rowsum_u8_list(const RowSumU8Params *d_jobs, const TileDesc *d_tiles, uint32_t n, const Geometry &g,
                                  bool flush, hipStream_t stream) {
+  if (g.matrix) return launch_rowsum_u8_matrix_list(d_jobs, d_tiles, n, g, stream);
   return dispatch(g, flush, [&](auto run, auto dpw, auto fl, auto pk) {
     hipLaunchKernelGGL((rowsum_u8_list<run.value, dpw.value, fl.value, pk.value>), dim3(n), dim3(64 * g.threads_d1),
                        g.lds_bytes, stream, d_jobs, d_tiles, n);
@@ -550,6 +504,7 @@ hipError_t launch_rowsum_u8_list(const RowSumU8Params *d_jobs, const TileDesc *d
 }
 
 hipError_t rowsum_u8_batch_occupancy(const Geometry &g, bool flush, int *per_cu) {
+  if (g.matrix) return rowsum_u8_matrix_batch_occupancy(g, per_cu);
   return dispatch(g, flush, [&](auto run, auto dpw, auto fl, auto pk) {
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, rowsum_u8_batch<run.value, dpw.value, fl.value, pk.value>,
                                                         (int)(64 * g.threads_d1), (size_t)g.lds_bytes);

@@ -31,6 +31,20 @@ dd_status hip_fail(hipError_t e, const char *what) {
 
 namespace {
 
+// Whether the matrix-core byte kernel sums `rows` rows faster than the vector
+// one, with `dms` DMs per wavefront and `windows` windows per row on average:
+// its products grow with the windows, the vector kernel's additions do not;
+// eight DMs share the operands that four read; above 257 rows the vector kernel
+// spills its 16-bit sums to 32 bits.  Measured (us, matrix against vector form,
+// each at its best shape): 1024 DMs x 24576 samples, 1.0 windows: 48 rows 45
+// and 45, 64 rows 53 and 56, 256 rows 144 and 175, 512 rows 264 and 399; 512
+// DMs, 256 rows: 1.4 windows 102 and 101, 2.0 windows 119 and 115; 1536 rows: 1.1
+// windows 444 and 632, 1.4 windows 543 and 633, 2.0 windows 657 and 635.
+bool matrix_is_faster(uint32_t rows, uint32_t dms, float windows) {
+  if (rows < 64) return false;
+  return windows <= (dms < 8 ? 1.1f : rows > 257 ? 1.6f : 1.25f);
+}
+
 uint32_t cps(const dd_plan *p) { return p->obs.nr_channels / p->obs.nr_subbands; }
 
 // Observation getters with the semantics stated in include/Observation.hpp.
@@ -88,6 +102,7 @@ dd_status build_integer(dd_plan *p, ShiftTable &t, const float *d_table, uint32_
   t.dms = dms;
   t.spread_cache.clear();
   t.pair_cache.clear();
+  t.window_cache.clear();
   t.pitch = roundup(std::max(dms, 1u), 64) + 64;
   DD_HIP(t.dev.allocate((size_t)rows * t.pitch));
   if (dms == 0 || rows == 0) {
@@ -158,7 +173,7 @@ dd_conf default_conf(dd_mode mode) {
     c.threads_d1 = 8;
     c.items_d0 = 16;
     c.items_d1 = 8;
-    c.unroll = 4;
+    c.unroll = 16;
     break;
   case DD_STEP_ONE:
     c.threads_d1 = 4;
@@ -266,6 +281,8 @@ dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry
   g.items_d1 = c.items_d1;
   g.packed = 0;
   g.pairs = 0;
+  g.matrix = 0;
+  g.wide = 0;
   g.unroll = c.unroll;
   // rows of floats: step two, and the single step and step one over float input
   const bool float_rows = mode == DD_STEP_TWO || p->input_bits == 32;
@@ -379,6 +396,7 @@ dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry
           g.packed = per > 1;
           g.unroll = unroll;
           g.lds_bytes = lds_of(unroll);
+          if (g.lds_bytes <= p->max_lds) set_byte_kernel(p, mode, c, ByteKernel::kByRule, g);
         }
       } else if (per > 1) {
         return fail(DD_ERR_CONFIGURATION, "packed input needs the pipelined kernel, whose row window is at most " +
@@ -400,12 +418,38 @@ dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry
   return DD_OK;
 }
 
+void set_byte_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, ByteKernel kernel, Geometry &g) {
+  if (g.staged != 1 || mode == DD_STEP_TWO || p->input_bits == 32) return;
+  const ShiftTable &t = mode == DD_SINGLE_STEP ? p->ish_single : p->ish_one;
+  const uint32_t tile = c.threads_d1 * c.items_d1;
+  const uint32_t slots = mode == DD_SINGLE_STEP ? p->obs.nr_channels : cps(p);
+  // vector form: rows | [2 buffers][rows per barrier][4 copies of a window] | DM words;
+  // matrix form: [1 raw][rows per barrier][windows] | rows | [2 buffers][rows per barrier][windows] | words of
+  // [2 buffers][rows per barrier, rounded up to 4, and 4 more].  Rows per barrier are capped at what fits in LDS
+  // a row is read as far as the widest of its four goes: past the last window by that row's spread
+  const uint32_t past = roundup(t.max_spread(c.items_d1), 16);
+  auto lds_of = [&](uint32_t u, bool matrix) {
+    if (matrix)
+      return 4 * (4 * slots + 3 * u * ((g.win + kU8MatrixReach) / 4) + 2 * (roundup(u, 4) + 4) * (tile + c.threads_d1)) + past;
+    return 4 * (roundup(2 * slots, 4) + 2 * u * g.win + 2 * u * tile);
+  };
+  const bool shaped = (c.items_d1 == 4 || c.items_d1 == 8) && g.win <= kU8MatrixWindow && lds_of(1, true) <= p->max_lds;
+  g.matrix = shaped && (kernel == ByteKernel::kMatrix ||
+                        (kernel == ByteKernel::kByRule && matrix_is_faster(slots, c.items_d1, t.mean_windows(c.items_d1))));
+  // one window takes the first DM's shift modulo 8, the spread and the block's 8 samples
+  g.wide = g.matrix && t.max_spread(c.items_d1) + 7 + 7 >= 32;
+  uint32_t unroll = std::min(c.unroll, kStagedSlotsPerWave * c.threads_d1);
+  while (unroll > 1 && lds_of(unroll, g.matrix) > p->max_lds) --unroll;
+  g.unroll = unroll;
+  g.lds_bytes = lds_of(unroll, g.matrix);
+}
+
 namespace {
 bool aligned16(const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 } // namespace
 
 dd_status prepare_single(dd_plan *plan, const dd_conf &c, const uint8_t *d_input, float *d_output,
-                         uint32_t first_sbeam, uint32_t nr_sbeams, U8Launch &L) {
+                         uint32_t first_sbeam, uint32_t nr_sbeams, U8Launch &L, ByteKernel kernel) {
   if (!plan || !d_input || !d_output) return fail(DD_ERR_INVALID_ARGUMENT, "null argument");
   if (plan->input_bits == 32) return fail(DD_ERR_INVALID_ARGUMENT, "the plan takes float input (dd_dedisperse_f32)");
   const dd_observation &o = plan->obs;
@@ -417,6 +461,9 @@ dd_status prepare_single(dd_plan *plan, const dd_conf &c, const uint8_t *d_input
     return fail(DD_ERR_INVALID_ARGUMENT, "dispersed batch shorter than samples + largest shift");
   dd_status s = geometry_of(plan, DD_SINGLE_STEP, c, L.g);
   if (s != DD_OK) return s;
+  // the matrix form's loads to LDS want the input at a dword
+  if ((reinterpret_cast<uintptr_t>(d_input) & 3) != 0) kernel = ByteKernel::kVector;
+  if (kernel != ByteKernel::kByRule) set_byte_kernel(plan, DD_SINGLE_STEP, c, kernel, L.g);
   RowSumU8Params &k = L.k;
   k = RowSumU8Params{};
   k.in = d_input;
@@ -462,7 +509,7 @@ dd_status prepare_single(dd_plan *plan, const dd_conf &c, const uint8_t *d_input
 }
 
 dd_status prepare_step_one(dd_plan *plan, const dd_conf &c, const uint8_t *d_input, float *d_intermediate,
-                           U8Launch &L) {
+                           U8Launch &L, ByteKernel kernel) {
   if (!plan || !d_input || !d_intermediate) return fail(DD_ERR_INVALID_ARGUMENT, "null argument");
   if (!plan->two_step) return fail(DD_ERR_INVALID_ARGUMENT, "plan has no subband path");
   if (plan->input_bits == 32)
@@ -473,6 +520,9 @@ dd_status prepare_step_one(dd_plan *plan, const dd_conf &c, const uint8_t *d_inp
     return fail(DD_ERR_INVALID_ARGUMENT, "dispersed batch shorter than samples + largest shift");
   dd_status s = geometry_of(plan, DD_STEP_ONE, c, L.g);
   if (s != DD_OK) return s;
+  // the matrix form's loads to LDS want the input at a dword
+  if ((reinterpret_cast<uintptr_t>(d_input) & 3) != 0) kernel = ByteKernel::kVector;
+  if (kernel != ByteKernel::kByRule) set_byte_kernel(plan, DD_STEP_ONE, c, kernel, L.g);
   RowSumU8Params &k = L.k;
   k = RowSumU8Params{};
   k.in = d_input;

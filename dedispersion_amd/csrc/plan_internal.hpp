@@ -70,6 +70,22 @@ struct ShiftTable {
     return m;
   }
   mutable std::vector<std::pair<uint32_t, uint32_t>> spread_cache;
+  // Mean number of 32-sample windows that the matrix-core byte kernel takes
+  // per row and wavefront of `dms` consecutive DMs: the first DM's shift is
+  // rounded down to 8 samples (3 on average) and an output block reaches 7
+  // samples past the last DM's (cached per DM count like max_spread).
+  float mean_windows(uint32_t dms) const {
+    for (auto &c : window_cache)
+      if (c.first == dms) return c.second;
+    uint64_t sum = 0, n = 0;
+    for (uint32_t r = 0; r < rows; ++r)
+      for (uint32_t d0 = 0; d0 < this->dms; d0 += dms, ++n)
+        sum += 1 + (uint64_t)(at(r, std::min(d0 + dms - 1, pitch - 1)) - at(r, d0) + 10) / 32;
+    const float mean = n ? (float)((double)sum / (double)n) : 1.0f;
+    window_cache.emplace_back(dms, mean);
+    return mean;
+  }
+  mutable std::vector<std::pair<uint32_t, float>> window_cache;
   // Most values that the shift difference of a row pair (2k, 2k + 1) takes
   // over the DMs of any tile of `tile` consecutive DMs, counted as the width
   // of its range (cached per tile size like max_spread).
@@ -136,6 +152,12 @@ dd_status hip_fail(hipError_t e, const char *what);
 
 // Geometry of a mode under a configuration; validates limits.
 dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry &g);
+// Which form of the staged byte kernel a launch takes: by the plan's own rule,
+// or one form for every job of a batch.
+enum class ByteKernel { kByRule, kVector, kMatrix };
+// Sets the form of a staged byte geometry (no effect on others, and where the
+// matrix form has no such shape) and the LDS that it needs.
+void set_byte_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, ByteKernel kernel, Geometry &g);
 
 // One prepared launch of a mode: kernel parameters, geometry and grid.
 struct U8Launch {
@@ -154,9 +176,10 @@ struct F32Launch {
 // (the checks and parameters of dd_dedisperse, dd_subband_step_one and
 // dd_subband_step_two).  n_tiles_x/y/n are set for every geometry.
 dd_status prepare_single(dd_plan *plan, const dd_conf &c, const uint8_t *d_input, float *d_output,
-                         uint32_t first_sbeam, uint32_t nr_sbeams, U8Launch &L);
+                         uint32_t first_sbeam, uint32_t nr_sbeams, U8Launch &L,
+                         ByteKernel kernel = ByteKernel::kByRule);
 dd_status prepare_step_one(dd_plan *plan, const dd_conf &c, const uint8_t *d_input, float *d_intermediate,
-                           U8Launch &L);
+                           U8Launch &L, ByteKernel kernel = ByteKernel::kByRule);
 dd_status prepare_step_two(dd_plan *plan, const dd_conf &c, const float *d_intermediate, float *d_output,
                            uint32_t first_sbeam, uint32_t nr_sbeams, F32Launch &L);
 // Step two over the uint16 sums that step one writes with out_u16 (a batch
