@@ -11,6 +11,7 @@
 // promising ones are timed; the exhaustive sweep stays the fallback.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <random>
@@ -26,76 +27,263 @@ using ddamd::set_error;
 
 constexpr uint32_t kMaxWidth = 256;
 
-// Y[r][j] = act(b[j] + sum_i X[r][i] W[i][j]) for r < n, j < dout.
-__global__ void dense_forward(const float *__restrict__ X, uint32_t n, uint32_t din, const float *__restrict__ W,
-                              const float *__restrict__ b, uint32_t dout, int relu, float *__restrict__ Y) {
-  const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (uint64_t)n * dout) return;
-  const uint32_t r = (uint32_t)(idx / dout), j = (uint32_t)(idx % dout);
-  const float *x = X + (uint64_t)r * din;
-  float acc = b[j];
-  for (uint32_t i = 0; i < din; ++i) acc += x[i] * W[(uint64_t)i * dout + j];
-  Y[idx] = relu ? fmaxf(acc, 0.0f) : acc;
+// The network's shape: dense layers 0 .. layers (the last has one unit).
+struct Shape {
+  uint32_t inputs, hidden, layers;
+  __host__ __device__ uint32_t fan_in(uint32_t l) const { return l == 0 ? inputs : hidden; }
+  __host__ __device__ uint32_t fan_out(uint32_t l) const { return l == layers ? 1 : hidden; }
+  __host__ __device__ uint32_t offset(uint32_t l) const {  // of layer l's weights; its biases follow
+    return l == 0 ? 0 : inputs * hidden + hidden + (l - 1) * (hidden * hidden + hidden);
+  }
+  // the same in LDS, where every row of weights is followed by an unused float
+  // so that neither a walk along a row nor one down a column meets bank conflicts
+  __host__ __device__ uint32_t lds_offset(uint32_t l) const {
+    return l == 0 ? 0 : inputs * (hidden + 1) + hidden + (l - 1) * (hidden * (hidden + 1) + hidden);
+  }
+  __host__ __device__ uint32_t lds_floats() const { return (lds_offset(layers) + 2 * hidden + 1 + 3) & ~3u; }
+};
+
+constexpr uint32_t kColumns = 16;       // columns of a weight matrix transposed through LDS at a time
+constexpr uint32_t kMaxGroups = 512;    // workgroups of the gradient pass (partial gradients)
+constexpr uint32_t kMaxLds = 64 * 1024;
+
+// A layer's weights W[i * ld + j] and biases, in LDS or in the parameter array.
+struct Layer {
+  const float *W, *b;
+  uint32_t ld;
+};
+
+template <bool RESIDENT>
+__device__ __forceinline__ Layer layer_of(const Shape &s, uint32_t l, const float *params, const float *weights) {
+  const uint32_t a = s.fan_in(l), b = s.fan_out(l);
+  if (RESIDENT) return Layer{weights + s.lds_offset(l), weights + s.lds_offset(l) + a * (b + 1), b + 1};
+  return Layer{params + s.offset(l), params + s.offset(l) + a * b, b};
 }
 
-// Output layer error of L = (1/n) sum_r (y_r - t_r)^2: G[r] = 2 (y_r - t_r) / n,
-// and the per-row squared error into E.
-__global__ void mse_error(const float *__restrict__ y, const float *__restrict__ t, uint32_t n, float *__restrict__ G,
-                          float *__restrict__ E) {
-  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  const float d = y[r] - t[r];
-  G[r] = 2.0f * d / (float)n;
-  E[r] = d * d;
+constexpr uint32_t kBatch = 8;  // reads sent for together, before any of them is used
+
+// All parameters to LDS: wavefronts take rows of weights (row a: the biases) and
+// lanes their columns.
+__device__ __forceinline__ void read_weights(const Shape &s, const float *__restrict__ params, float *weights) {
+  const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64, waves = blockDim.x / 64;
+  for (uint32_t l = 0; l <= s.layers; ++l) {
+    const uint32_t a = s.fan_in(l), b = s.fan_out(l);
+    const float *from = params + s.offset(l);
+    float *to = weights + s.lds_offset(l);
+    for (uint32_t j = lane; j < b; j += 64)
+      for (uint32_t i0 = wave; i0 <= a; i0 += waves * kBatch) {
+        float v[kBatch];
+#pragma unroll
+        for (uint32_t k = 0; k < kBatch; ++k) v[k] = from[min(i0 + k * waves, a) * b + j];
+#pragma unroll
+        for (uint32_t k = 0; k < kBatch; ++k)
+          if (i0 + k * waves <= a) to[(i0 + k * waves) * (b + 1) + j] = v[k];
+      }
+  }
 }
 
-// loss = (1/n) sum E, one workgroup of 256 threads.
-__global__ void mean_of(const float *__restrict__ E, uint32_t n, float *__restrict__ out) {
-  __shared__ float part[256];
-  float s = 0.0f;
-  for (uint32_t r = threadIdx.x; r < n; r += blockDim.x) s += E[r];
-  part[threadIdx.x] = s;
+// acc += sum over c < n, in order, of e[c * R .. + 3] w[c * ld].
+template <uint32_t R>
+__device__ __forceinline__ void add_products(float4 &acc, const float *e, const float *w, uint32_t n, uint32_t ld) {
+  auto add = [&](const float4 &x, float y) {
+    acc.x += x.x * y;
+    acc.y += x.y * y;
+    acc.z += x.z * y;
+    acc.w += x.w * y;
+  };
+  uint32_t c = 0;
+  for (; c + kBatch <= n; c += kBatch) {
+    float4 x[kBatch];
+    float y[kBatch];
+#pragma unroll
+    for (uint32_t k = 0; k < kBatch; ++k) {
+      y[k] = w[(c + k) * ld];
+      x[k] = *reinterpret_cast<const float4 *>(e + (c + k) * R);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // the scheduler would read each next to its use
+#pragma unroll
+    for (uint32_t k = 0; k < kBatch; ++k) add(x[k], y[k]);
+  }
+  for (; c < n; ++c) add(*reinterpret_cast<const float4 *>(e + c * R), w[c * ld]);
+}
+
+// One layer over R rows held unit by unit (in[i * R + r]): out[j][r] = act(b[j]
+// + sum over i, in order, of in[i][r] W[i][j]); a thread takes four rows of a
+// unit, and consecutive threads consecutive units.
+template <uint32_t R>
+__device__ __forceinline__ void dense(const Layer &y, uint32_t din, uint32_t dout, bool relu, const float *in, float *out) {
+  for (uint32_t idx = threadIdx.x; idx < dout * (R / 4); idx += blockDim.x) {
+    const uint32_t j = idx % dout, q = 4 * (idx / dout);
+    const float bias = y.b[j];
+    float4 acc = make_float4(bias, bias, bias, bias);
+    add_products<R>(acc, in + q, y.W + j, din, y.ld);
+    if (relu) acc = make_float4(fmaxf(acc.x, 0.0f), fmaxf(acc.y, 0.0f), fmaxf(acc.z, 0.0f), fmaxf(acc.w, 0.0f));
+    *reinterpret_cast<float4 *>(out + j * R + q) = acc;
+  }
+}
+
+// Rows r0 .. r0 + R - 1 of X (n x inputs) to in[i * R + r]; zeros past row n.
+template <uint32_t R>
+__device__ __forceinline__ void read_rows(const float *__restrict__ X, uint32_t n, uint32_t inputs, uint64_t r0, float *in) {
+  for (uint32_t idx = threadIdx.x; idx < inputs * R; idx += blockDim.x) {
+    const uint32_t r = idx / inputs, i = idx % inputs;
+    in[i * R + r] = r0 + r < n ? X[(r0 + r) * inputs + i] : 0.0f;
+  }
+}
+
+// The whole network over R rows per workgroup; activations stay in LDS (two
+// buffers in turn), as do the weights where they fit (RESIDENT).
+template <uint32_t R, bool RESIDENT>
+__global__ void __launch_bounds__(256) mlp_forward(const Shape s, const float *__restrict__ X, uint32_t n,
+                                                   const float *__restrict__ params, float *__restrict__ Y) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const uint32_t width = s.inputs > s.hidden ? s.inputs : s.hidden;
+  float *in = lds, *out = lds + width * R;
+  const float *weights = lds + 2 * width * R;
+  if (RESIDENT) read_weights(s, params, lds + 2 * width * R);
+  const uint64_t r0 = (uint64_t)blockIdx.x * R;
+  read_rows<R>(X, n, s.inputs, r0, in);
   __syncthreads();
-  for (uint32_t w = blockDim.x / 2; w > 0; w /= 2) {
-    if (threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
+  for (uint32_t l = 0; l <= s.layers; ++l) {
+    dense<R>(layer_of<RESIDENT>(s, l, params, weights), s.fan_in(l), s.fan_out(l), l < s.layers, in, out);
+    __syncthreads();
+    float *t = in;
+    in = out;
+    out = t;
+  }
+  if (threadIdx.x < R && r0 + threadIdx.x < n) Y[r0 + threadIdx.x] = in[threadIdx.x];
+}
+
+// Forward and backward pass of L = (1/n) sum_r (y_r - t_r)^2 over R rows at a
+// time.  Activations and errors stay in LDS.  Workgroup g takes row blocks g, g
+// + gridDim.x, ... and leaves its part of dL/dparams in part[g * (count + 1)],
+// followed by its sum of squared errors.
+//
+// A pass over 2880 rows of the tuner's 9217 parameters took 2860 us as one
+// launch per layer and operation, with one thread per weight walking all rows in
+// 17 workgroups; as this pass and the sum of its parts it takes 39 us (70 with the
+// weights read through the caches in every layer).  It is bound by the latency of
+// one workgroup's chain of layers, so a workgroup takes as few rows as still
+// share a weight read.
+template <uint32_t R, bool RESIDENT>
+__global__ void __launch_bounds__(256) mlp_gradient(const Shape s, const float *__restrict__ X,
+                                                    const float *__restrict__ T, uint32_t n,
+                                                    const float *__restrict__ params, uint32_t count,
+                                                    float *__restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float *act = lds;  // the input rows, then every hidden layer's output
+  float *G = act + (s.inputs + s.layers * s.hidden) * R, *GX = G + s.hidden * R;
+  // all weights, or [hidden][kColumns + 1] of a layer's; the squares
+  float *weights = GX + s.hidden * R, *cols = weights;
+  float *squares = weights + (RESIDENT ? s.lds_floats() : s.hidden * (kColumns + 1));
+  if (RESIDENT) read_weights(s, params, weights);
+  float *mine = part + (uint64_t)blockIdx.x * (count + 1);
+  auto input_of = [&](uint32_t l) { return act + (l == 0 ? 0 : (s.inputs + (l - 1) * s.hidden) * R); };
+  bool first = true;
+  for (uint64_t r0 = (uint64_t)blockIdx.x * R; r0 < n; r0 += (uint64_t)gridDim.x * R, first = false) {
+    read_rows<R>(X, n, s.inputs, r0, act);
+    __syncthreads();
+    for (uint32_t l = 0; l <= s.layers; ++l) {
+      dense<R>(layer_of<RESIDENT>(s, l, params, weights), s.fan_in(l), s.fan_out(l), l < s.layers, input_of(l),
+               l < s.layers ? input_of(l + 1) : GX);
+      __syncthreads();
+    }
+    // the output's error 2 (y - t) / n, and the squares
+    if (threadIdx.x < R) {
+      const bool row = r0 + threadIdx.x < n;
+      const float d = row ? GX[threadIdx.x] - T[r0 + threadIdx.x] : 0.0f;
+      G[threadIdx.x] = 2.0f * d / (float)n;
+      squares[threadIdx.x] = d * d;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      float e = first ? 0.0f : mine[count];
+      for (uint32_t r = 0; r < R; ++r) e += squares[r];
+      mine[count] = e;
+    }
+    for (uint32_t l = s.layers + 1; l-- > 0;) {
+      const uint32_t a = s.fan_in(l), b = s.fan_out(l);
+      const Layer y = layer_of<RESIDENT>(s, l, params, weights);
+      const float *in = input_of(l);
+      // weights W[i][j] and, as row i = a, the biases
+      uint32_t held = ~0u;
+      float4 g[R / 4];
+      for (uint32_t idx = threadIdx.x; idx < (a + 1) * b; idx += blockDim.x) {
+        const uint32_t i = idx / b, j = idx % b;
+        if (j != held) {
+          held = j;
+#pragma unroll
+          for (uint32_t q = 0; q < R / 4; ++q) g[q] = *reinterpret_cast<const float4 *>(G + j * R + 4 * q);
+        }
+        float sum = 0.0f;
+#pragma unroll
+        for (uint32_t q = 0; q < R / 4; ++q) {
+          const float4 x = i < a ? *reinterpret_cast<const float4 *>(in + i * R + 4 * q) : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+          sum += x.x * g[q].x;
+          sum += x.y * g[q].y;
+          sum += x.z * g[q].z;
+          sum += x.w * g[q].w;
+        }
+        float *slot = mine + s.offset(l) + idx;
+        *slot = first ? sum : *slot + sum;
+      }
+      if (l == 0) break;
+      // the layer input's error, through the ReLU of the layer below: GX[i][r] =
+      // (in[i][r] > 0) * sum over j, in order, of G[j][r] W[i][j].  Threads take
+      // consecutive i, whose weights lie a row apart: where they are not in LDS,
+      // they come through it, kColumns columns at a time.
+      const uint32_t step = RESIDENT ? b : kColumns;
+      for (uint32_t j0 = 0; j0 < b; j0 += step) {
+        const uint32_t nj = b - j0 < step ? b - j0 : step;
+        if (!RESIDENT) {
+          __syncthreads();
+          for (uint32_t idx = threadIdx.x; idx < a * kColumns; idx += blockDim.x) {
+            const uint32_t i = idx / kColumns, c = idx % kColumns;
+            if (c < nj) cols[i * (kColumns + 1) + c] = y.W[i * y.ld + j0 + c];
+          }
+          __syncthreads();
+        }
+        for (uint32_t idx = threadIdx.x; idx < a * (R / 4); idx += blockDim.x) {
+          const uint32_t i = idx % a, q = 4 * (idx / a);
+          const float *row = RESIDENT ? weights + s.lds_offset(l) + i * (b + 1) : cols + i * (kColumns + 1);
+          float4 *gx = reinterpret_cast<float4 *>(GX + i * R + q);
+          float4 acc = j0 == 0 ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : *gx;
+          add_products<R>(acc, G + j0 * R + q, row, nj, 1);
+          if (j0 + nj == b) {
+            const float4 h = *reinterpret_cast<const float4 *>(in + i * R + q);
+            acc = make_float4(h.x <= 0.0f ? 0.0f : acc.x, h.y <= 0.0f ? 0.0f : acc.y, h.z <= 0.0f ? 0.0f : acc.z,
+                              h.w <= 0.0f ? 0.0f : acc.w);
+          }
+          *gx = acc;
+        }
+      }
+      __syncthreads();
+      float *t = G;
+      G = GX;
+      GX = t;
+    }
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[0] = part[0] / (float)n;
 }
 
-// dW[i][j] = sum_r X[r][i] G[r][j]; db[j] = sum_r G[r][j].  One thread per
-// weight (and per bias, the extra row i = din).
-__global__ void dense_weight_grad(const float *__restrict__ X, const float *__restrict__ G, uint32_t n, uint32_t din,
-                                  uint32_t dout, float *__restrict__ dW, float *__restrict__ db) {
-  const uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (din + 1) * dout) return;
-  const uint32_t i = idx / dout, j = idx % dout;
-  float acc = 0.0f;
-  if (i < din) {
-    for (uint32_t r = 0; r < n; ++r) acc += X[(uint64_t)r * din + i] * G[(uint64_t)r * dout + j];
-    dW[(uint64_t)i * dout + j] = acc;
-  } else {
-    for (uint32_t r = 0; r < n; ++r) acc += G[(uint64_t)r * dout + j];
-    db[j] = acc;
+// grad[k] = the sum of the workgroups' parts, four threads per parameter; the
+// element past the last parameter is the loss.
+__global__ void __launch_bounds__(256) mlp_sum_parts(const float *__restrict__ part, uint32_t groups, uint32_t count,
+                                                     uint32_t n, float *__restrict__ grad, float *__restrict__ loss) {
+  __shared__ float sums[4][64];
+  const uint32_t lane = threadIdx.x % 64, seg = threadIdx.x / 64, k = blockIdx.x * 64 + lane;
+  float sum = 0.0f;
+  if (k <= count) {
+#pragma unroll 8
+    for (uint32_t g = seg; g < groups; g += 4) sum += part[(uint64_t)g * (count + 1) + k];
   }
-}
-
-// Error at the layer input, through the ReLU of the layer below:
-// GX[r][i] = (H[r][i] > 0) * sum_j G[r][j] W[i][j].
-__global__ void dense_input_grad(const float *__restrict__ G, const float *__restrict__ W, const float *__restrict__ H,
-                                 uint32_t n, uint32_t din, uint32_t dout, float *__restrict__ GX) {
-  const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (uint64_t)n * din) return;
-  const uint32_t r = (uint32_t)(idx / din), i = (uint32_t)(idx % din);
-  if (H[idx] <= 0.0f) {
-    GX[idx] = 0.0f;
-    return;
+  sums[seg][lane] = sum;
+  __syncthreads();
+  if (seg == 0 && k <= count) {
+    const float all = (sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane]);
+    if (k < count) grad[k] = all;
+    else loss[0] = all / (float)n;
   }
-  const float *g = G + (uint64_t)r * dout;
-  const float *w = W + (uint64_t)i * dout;
-  float acc = 0.0f;
-  for (uint32_t j = 0; j < dout; ++j) acc += g[j] * w[j];
-  GX[idx] = acc;
 }
 
 // Adam (Kingma and Ba, 2015) with bias correction factors c1 = 1 - beta1^t,
@@ -118,33 +306,16 @@ inline uint32_t blocks_for(uint64_t n, uint32_t threads) { return (uint32_t)((n 
 } // namespace
 
 struct dd_mlp {
-  uint32_t inputs = 0, hidden = 0, layers = 0;  // hidden layers
-  std::vector<uint32_t> fan_in, fan_out;         // per dense layer (layers + 1)
-  std::vector<size_t> w_off, b_off;              // offsets into the flat parameter array
+  Shape shape{};
   size_t count = 0;
-  float *params = nullptr, *m = nullptr, *v = nullptr;
+  float *params = nullptr, *m = nullptr, *v = nullptr, *grad_tmp = nullptr;
   uint32_t step = 0;
-  // activations / errors for the last n rows
-  uint32_t cap = 0;
-  std::vector<float *> act;   // act[0] unused (the input), act[l] = output of layer l-1 (n x fan_out)
-  float *err_a = nullptr, *err_b = nullptr, *sq = nullptr, *grad_tmp = nullptr, *loss_tmp = nullptr;
+  // parts of the gradient, one per workgroup, and the losses of a training run
+  float *part = nullptr, *losses = nullptr;
+  uint32_t part_groups = 0, losses_cap = 0;
 
   ~dd_mlp() {
-    (void)hipFree(params);
-    (void)hipFree(m);
-    (void)hipFree(v);
-    release_rows();
-    (void)hipFree(grad_tmp);
-    (void)hipFree(loss_tmp);
-  }
-  void release_rows() {
-    for (float *p : act) (void)hipFree(p);
-    act.clear();
-    (void)hipFree(err_a);
-    (void)hipFree(err_b);
-    (void)hipFree(sq);
-    err_a = err_b = sq = nullptr;
-    cap = 0;
+    for (float *p : {params, m, v, grad_tmp, part, losses}) (void)hipFree(p);
   }
 };
 
@@ -161,57 +332,62 @@ dd_status fail_mlp(dd_status s, const std::string &msg) {
     if (e_ != hipSuccess) return fail_mlp(DD_ERR_HIP, std::string(#call) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-dd_status reserve_rows(dd_mlp *net, uint32_t n) {
-  if (n <= net->cap) return DD_OK;
-  net->release_rows();
-  net->act.assign(net->layers + 2, nullptr);
-  for (uint32_t l = 0; l <= net->layers; ++l)
-    MLP_HIP(hipMalloc(reinterpret_cast<void **>(&net->act[l + 1]), (size_t)n * net->fan_out[l] * sizeof(float)));
-  const uint32_t widest = std::max(net->hidden, net->inputs);
-  MLP_HIP(hipMalloc(reinterpret_cast<void **>(&net->err_a), (size_t)n * widest * sizeof(float)));
-  MLP_HIP(hipMalloc(reinterpret_cast<void **>(&net->err_b), (size_t)n * widest * sizeof(float)));
-  MLP_HIP(hipMalloc(reinterpret_cast<void **>(&net->sq), (size_t)n * sizeof(float)));
-  net->cap = n;
+// LDS of a gradient and of a forward pass over R rows per workgroup.
+uint32_t gradient_lds(const Shape &s, uint32_t R, bool resident) {
+  return 4 * ((s.inputs + s.layers * s.hidden + 2 * s.hidden + 1) * R +
+              (resident ? s.lds_floats() : s.hidden * (kColumns + 1)));
+}
+uint32_t forward_lds(const Shape &s, uint32_t R, bool resident) {
+  return 4 * (2 * std::max(s.inputs, s.hidden) * R + (resident ? s.lds_floats() : 0));
+}
+
+// The weights are kept in LDS where 16 rows' activations fit beside them (up to
+// three hidden layers of 64, or one of 100); else a workgroup takes four rows.
+bool resident(const Shape &s) { return gradient_lds(s, 16, true) <= kMaxLds; }
+uint32_t gradient_rows(const Shape &s) { return resident(s) ? 16 : 4; }
+
+uint32_t gradient_groups(const Shape &s, uint32_t n) {
+  return std::min(blocks_for(n, gradient_rows(s)), kMaxGroups);
+}
+
+dd_status reserve(float *&p, uint32_t &have, uint32_t want, size_t each) {
+  if (want <= have) return DD_OK;
+  (void)hipFree(p);
+  p = nullptr;
+  have = 0;
+  MLP_HIP(hipMalloc(reinterpret_cast<void **>(&p), (size_t)want * each * sizeof(float)));
+  have = want;
   return DD_OK;
 }
 
-dd_status forward(dd_mlp *net, const float *d_x, uint32_t n, hipStream_t s) {
-  const float *in = d_x;
-  for (uint32_t l = 0; l <= net->layers; ++l) {
-    const uint32_t a = net->fan_in[l], b = net->fan_out[l];
-    const int relu = l < net->layers ? 1 : 0;
-    hipLaunchKernelGGL(dense_forward, dim3(blocks_for((uint64_t)n * b, 256)), dim3(256), 0, s, in, n, a,
-                       net->params + net->w_off[l], net->params + net->b_off[l], b, relu, net->act[l + 1]);
-    MLP_HIP(hipGetLastError());
-    in = net->act[l + 1];
-  }
+dd_status reserve_parts(dd_mlp *net, uint32_t n) {
+  return reserve(net->part, net->part_groups, gradient_groups(net->shape, n), net->count + 1);
+}
+
+dd_status forward(dd_mlp *net, const float *d_x, uint32_t n, float *d_y, hipStream_t s) {
+  const Shape &sh = net->shape;
+  if (resident(sh))
+    hipLaunchKernelGGL((mlp_forward<16, true>), dim3(blocks_for(n, 16)), dim3(256), forward_lds(sh, 16, true), s, sh, d_x,
+                       n, net->params, d_y);
+  else
+    hipLaunchKernelGGL((mlp_forward<4, false>), dim3(blocks_for(n, 4)), dim3(256), forward_lds(sh, 4, false), s, sh, d_x,
+                       n, net->params, d_y);
+  MLP_HIP(hipGetLastError());
   return DD_OK;
 }
 
 dd_status loss_grad(dd_mlp *net, const float *d_x, const float *d_t, uint32_t n, float *d_loss, float *d_grad,
                     hipStream_t s) {
-  dd_status st = forward(net, d_x, n, s);
-  if (st != DD_OK) return st;
-  const uint32_t L = net->layers;
-  hipLaunchKernelGGL(mse_error, dim3(blocks_for(n, 256)), dim3(256), 0, s, net->act[L + 1], d_t, n, net->err_a,
-                     net->sq);
+  const Shape &sh = net->shape;
+  const uint32_t groups = gradient_groups(sh, n);
+  const bool keep = resident(sh);
+  auto kernel = keep ? mlp_gradient<16, true> : mlp_gradient<4, false>;
+  hipLaunchKernelGGL(kernel, dim3(groups), dim3(256), gradient_lds(sh, gradient_rows(sh), keep), s, sh, d_x, d_t, n,
+                     net->params, (uint32_t)net->count, net->part);
   MLP_HIP(hipGetLastError());
-  hipLaunchKernelGGL(mean_of, dim3(1), dim3(256), 0, s, net->sq, n, d_loss);
+  hipLaunchKernelGGL(mlp_sum_parts, dim3(blocks_for(net->count + 1, 64)), dim3(256), 0, s, net->part, groups,
+                     (uint32_t)net->count, n, d_grad, d_loss);
   MLP_HIP(hipGetLastError());
-  float *G = net->err_a, *GX = net->err_b;
-  for (int l = (int)L; l >= 0; --l) {
-    const uint32_t a = net->fan_in[l], b = net->fan_out[l];
-    const float *X = l == 0 ? d_x : net->act[l];
-    hipLaunchKernelGGL(dense_weight_grad, dim3(blocks_for((uint64_t)(a + 1) * b, 256)), dim3(256), 0, s, X, G, n, a,
-                       b, d_grad + net->w_off[l], d_grad + net->b_off[l]);
-    MLP_HIP(hipGetLastError());
-    if (l > 0) {
-      hipLaunchKernelGGL(dense_input_grad, dim3(blocks_for((uint64_t)n * a, 256)), dim3(256), 0, s, G,
-                         net->params + net->w_off[l], net->act[l], n, a, b, GX);
-      MLP_HIP(hipGetLastError());
-      std::swap(G, GX);
-    }
-  }
   return DD_OK;
 }
 
@@ -237,25 +413,13 @@ dd_status dd_mlp_create(dd_mlp **out, uint32_t inputs, uint32_t hidden, uint32_t
       hidden_layers > 8)
     return fail_mlp(DD_ERR_INVALID_ARGUMENT, "network shape out of range");
   dd_mlp *net = new dd_mlp();
-  net->inputs = inputs;
-  net->hidden = hidden;
-  net->layers = hidden_layers;
-  size_t off = 0;
-  for (uint32_t l = 0; l <= hidden_layers; ++l) {
-    const uint32_t a = l == 0 ? inputs : hidden, b = l == hidden_layers ? 1 : hidden;
-    net->fan_in.push_back(a);
-    net->fan_out.push_back(b);
-    net->w_off.push_back(off);
-    off += (size_t)a * b;
-    net->b_off.push_back(off);
-    off += b;
-  }
+  net->shape = Shape{inputs, hidden, hidden_layers};
+  const size_t off = net->shape.offset(hidden_layers) + hidden + 1;
   net->count = off;
   hipError_t e = hipMalloc(reinterpret_cast<void **>(&net->params), off * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&net->m), off * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&net->v), off * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&net->grad_tmp), off * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&net->loss_tmp), sizeof(float));
   if (e == hipSuccess) e = hipMemset(net->params, 0, off * sizeof(float));
   if (e == hipSuccess) e = hipMemset(net->m, 0, off * sizeof(float));
   if (e == hipSuccess) e = hipMemset(net->v, 0, off * sizeof(float));
@@ -298,10 +462,11 @@ dd_status dd_mlp_init(dd_mlp *net, uint64_t seed) {
   // He-uniform weights (bound sqrt(6 / fan_in)), zero biases.
   std::mt19937_64 rng(seed);
   std::vector<float> p(net->count, 0.0f);
-  for (uint32_t l = 0; l <= net->layers; ++l) {
-    const float bound = std::sqrt(6.0f / (float)net->fan_in[l]);
+  for (uint32_t l = 0; l <= net->shape.layers; ++l) {
+    const uint32_t a = net->shape.fan_in(l), b = net->shape.fan_out(l);
+    const float bound = std::sqrt(6.0f / (float)a);
     std::uniform_real_distribution<float> u(-bound, bound);
-    for (size_t k = 0; k < (size_t)net->fan_in[l] * net->fan_out[l]; ++k) p[net->w_off[l] + k] = u(rng);
+    for (size_t k = 0; k < (size_t)a * b; ++k) p[net->shape.offset(l) + k] = u(rng);
   }
   return dd_mlp_set_params(net, p.data());
 }
@@ -309,19 +474,14 @@ dd_status dd_mlp_init(dd_mlp *net, uint64_t seed) {
 dd_status dd_mlp_forward(dd_mlp *net, const float *d_x, uint32_t n, float *d_y, void *stream) {
   if (!net || !d_x || !d_y) return fail_mlp(DD_ERR_INVALID_ARGUMENT, "null argument");
   if (n == 0) return DD_OK;
-  dd_status s = reserve_rows(net, n);
-  if (s == DD_OK) s = forward(net, d_x, n, (hipStream_t)stream);
-  if (s != DD_OK) return s;
-  MLP_HIP(hipMemcpyAsync(d_y, net->act[net->layers + 1], (size_t)n * sizeof(float), hipMemcpyDeviceToDevice,
-                         (hipStream_t)stream));
-  return DD_OK;
+  return forward(net, d_x, n, d_y, (hipStream_t)stream);
 }
 
 dd_status dd_mlp_loss_grad(dd_mlp *net, const float *d_x, const float *d_target, uint32_t n, float *d_loss,
                            float *d_grad, void *stream) {
   if (!net || !d_x || !d_target || !d_loss || !d_grad || n == 0)
     return fail_mlp(DD_ERR_INVALID_ARGUMENT, "invalid argument");
-  dd_status s = reserve_rows(net, n);
+  dd_status s = reserve_parts(net, n);
   return s != DD_OK ? s : loss_grad(net, d_x, d_target, n, d_loss, d_grad, (hipStream_t)stream);
 }
 
@@ -333,15 +493,18 @@ dd_status dd_mlp_adam_step(dd_mlp *net, const float *d_grad, float lr, void *str
 dd_status dd_mlp_train(dd_mlp *net, const float *d_x, const float *d_target, uint32_t n, uint32_t steps, float lr,
                        float *losses, void *stream) {
   if (!net || !d_x || !d_target || n == 0) return fail_mlp(DD_ERR_INVALID_ARGUMENT, "invalid argument");
-  dd_status s = reserve_rows(net, n);
+  dd_status s = reserve_parts(net, n);
+  // the losses stay on the device until the run is over
+  if (s == DD_OK) s = reserve(net->losses, net->losses_cap, std::max(steps, 1u), 1);
   if (s != DD_OK) return s;
   hipStream_t st = (hipStream_t)stream;
   for (uint32_t k = 0; k < steps; ++k) {
-    s = loss_grad(net, d_x, d_target, n, net->loss_tmp, net->grad_tmp, st);
+    s = loss_grad(net, d_x, d_target, n, net->losses + k, net->grad_tmp, st);
     if (s == DD_OK) s = adam(net, net->grad_tmp, lr, st);
     if (s != DD_OK) return s;
-    if (losses) MLP_HIP(hipMemcpyAsync(losses + k, net->loss_tmp, sizeof(float), hipMemcpyDeviceToHost, st));
   }
+  if (losses && steps)
+    MLP_HIP(hipMemcpyAsync(losses, net->losses, (size_t)steps * sizeof(float), hipMemcpyDeviceToHost, st));
   MLP_HIP(hipStreamSynchronize(st));
   return DD_OK;
 }
