@@ -157,6 +157,7 @@ template <typename L> void merge_geometry(KindQueue &k, const L &launch, bool fi
     k.g.win = std::max(k.g.win, launch.g.win);
     k.g.packed |= launch.g.packed;
     k.g.wide |= launch.g.wide;
+    k.g.many |= launch.g.many;
   }
 }
 

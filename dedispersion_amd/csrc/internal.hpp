@@ -149,6 +149,7 @@ struct Geometry {
   uint32_t pairs;      // 1 = the paired uint16 step two (kernels_u16_pairs.hip)
   uint32_t matrix;     // 1 = the matrix-core form of the staged kernel (kernels_u8_matrix.hip)
   uint32_t wide;       // 1 = ... whose rows may take more than one window
+  uint32_t many;       // 1 = the staged float kernel for slices of more than kF32Rows rows
 };
 
 // Launchers (kernels_u8.hip / kernels_f32.hip).  Return hipSuccess or the
@@ -230,6 +231,9 @@ constexpr uint32_t kU8MatrixWindow = 2048;  // widest row window that it stages 
 constexpr uint32_t kStagedSlotsPerWave = 2;  // rows staged per wavefront per group
 constexpr uint32_t kU8StagedChunks = 2;      // 16-byte staging loads per lane per row (window <= 2 KiB)
 inline uint32_t f32_staged_chunks(uint32_t run) { return run / 4 + 1; }
+// The staged float kernel lists a slice's rows in LDS; more rows than this are
+// listed this many at a time.
+constexpr uint32_t kF32Rows = 2048;
 
 // Table kernels (tables.hip).
 struct ShiftFormula {

@@ -160,38 +160,6 @@ dd_status rebuild_live(dd_plan *p) {
   return DD_OK;
 }
 
-// Defaults: the fastest configurations of exhaustive sweeps on MI355X of the
-// ARTS layouts -- the single step (1536 channels, 2048 DMs, 24576 samples)
-// and the two-step path (32 subbands, 64 coarse x 32 fine DMs).
-dd_conf default_conf(dd_mode mode) {
-  dd_conf c{};
-  c.threads_d0 = 64;
-  c.split_batches = 0;
-  c.local = 1;
-  switch (mode) {
-  case DD_SINGLE_STEP:
-    c.threads_d1 = 8;
-    c.items_d0 = 16;
-    c.items_d1 = 8;
-    c.unroll = 16;
-    break;
-  case DD_STEP_ONE:
-    c.threads_d1 = 4;
-    c.items_d0 = 16;
-    c.items_d1 = 8;
-    c.unroll = 4;
-    break;
-  default:
-    c.threads_d1 = 8;
-    c.items_d0 = 8;
-    c.items_d1 = 4;
-    c.unroll = 8;
-    c.local = 2;
-    break;
-  }
-  return c;
-}
-
 // Pattern records of the single step for DM tiles of kFactoredDMs DMs and
 // blocks of four live channels (layout in internal.hpp).  fact_ok is false
 // when a record would need more than kFactoredMaxPatterns patterns or an
@@ -283,6 +251,7 @@ dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry
   g.pairs = 0;
   g.matrix = 0;
   g.wide = 0;
+  g.many = 0;
   g.unroll = c.unroll;
   // rows of floats: step two, and the single step and step one over float input
   const bool float_rows = mode == DD_STEP_TWO || p->input_bits == 32;
@@ -356,15 +325,16 @@ dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry
       g.win = roundup(ts + t.max_spread(tile), 4);
       g.lds_bytes = c.unroll * g.win * 4;
       if (stageable && g.win / 4 <= 64 * f32_staged_chunks(c.items_d0)) {
-        // rows (row | beam, delay) of a slice | [2 buffers][unroll rows][win] | DM offsets;
+        // [2 buffers][unroll rows][4 copies][win] | rows of a slice | DM addresses;
         // rows staged per barrier are capped at what fits in LDS
         const uint32_t slots = mode == DD_STEP_TWO ? p->obs.nr_subbands
                                : mode == DD_SINGLE_STEP ? p->obs.nr_channels : cps(p);
-        auto lds_of = [&](uint32_t u) { return 4 * (roundup(2 * slots, 4) + 2 * u * g.win + 2 * u * tile); };
+        auto lds_of = [&](uint32_t u) { return 4 * (4 * std::min(slots, kF32Rows) + 8 * u * g.win + 2 * u * tile); };
         uint32_t unroll = c.unroll;
         while (unroll > 1 && lds_of(unroll) > p->max_lds) --unroll;
         if (lds_of(unroll) <= p->max_lds) {
           g.staged = 1;
+          g.many = slots > kF32Rows;
           g.unroll = unroll;
           g.lds_bytes = lds_of(unroll);
         }
@@ -442,6 +412,66 @@ void set_byte_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, ByteKerne
   while (unroll > 1 && lds_of(unroll, g.matrix) > p->max_lds) --unroll;
   g.unroll = unroll;
   g.lds_bytes = lds_of(unroll, g.matrix);
+}
+
+namespace {
+
+dd_conf conf_of(uint32_t wavefronts, uint32_t items_d0, uint32_t items_d1, uint32_t unroll) {
+  dd_conf c{};
+  c.threads_d0 = 64;
+  c.threads_d1 = wavefronts;
+  c.items_d0 = items_d0;
+  c.items_d1 = items_d1;
+  c.unroll = unroll;
+  c.local = 1;
+  return c;
+}
+
+// Step two's shape for a plan's sizes, for a plan without a caller's configuration.
+// Measured on MI355X over 32 subbands, 8-128 coarse and 16-32 fine DMs and
+// 4000-32768 samples.
+dd_conf step_two_conf(const dd_plan *p) {
+  const dd_observation &o = p->obs;
+  const dd_sizes &z = p->sizes;
+  int cus = 256;
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device);
+  // few rows (subbands) and much output: small groups of rows and many
+  // workgroups per compute unit, once there are several for each
+  const uint32_t d1 = o.nr_dms <= 16 ? 2 : o.nr_dms <= 32 ? 4 : 8;
+  const uint64_t tiles = (uint64_t)((z.nr_samples + 511) / 512) * ((o.nr_dms + 8 * d1 - 1) / (8 * d1)) *
+                         o.nr_synthesized_beams * o.nr_dms_subbanding;
+  if (tiles >= 10ull * cus && d1 == 4) return conf_of(8, 16, 4, 2);
+  if (tiles >= 4ull * cus) return conf_of(8, 8, d1, 2);
+  return conf_of(8, tiles >= (uint64_t)cus * 3 / 4 ? 8 : 4, d1, 8);
+}
+
+// The shapes that every plan started from.  What they refuse (row windows too
+// wide for packed rows) stays refused, and a plan whose windows fit them but not
+// the shape of its sizes runs them.
+dd_conf plain_conf(dd_mode mode) {
+  switch (mode) {
+  case DD_SINGLE_STEP: return conf_of(8, 16, 8, 16);
+  case DD_STEP_ONE: return conf_of(4, 16, 8, 4);
+  default: return conf_of(8, 8, 4, 8);
+  }
+}
+
+} // namespace
+
+void set_default_confs(dd_plan *p) {
+  for (int m = 0; m < 3; ++m) {
+    if (p->conf_set[m]) continue;
+    const dd_mode mode = (dd_mode)m;
+    p->conf[m] = plain_conf(mode);
+    if (mode != DD_SINGLE_STEP && !p->two_step) continue;
+    Geometry plain, g;
+    if (mode != DD_STEP_TWO) continue;
+    const dd_conf c = step_two_conf(p);
+    if (geometry_of(p, mode, c, g) != DD_OK) continue;
+    const bool packed = mode != DD_STEP_TWO && p->input_bits < 8;
+    if ((g.staged && !packed) || (geometry_of(p, mode, p->conf[m], plain) == DD_OK && g.staged >= plain.staged))
+      p->conf[m] = c;
+  }
 }
 
 namespace {
@@ -700,6 +730,7 @@ dd_status prepare_single_f32(dd_plan *plan, const dd_conf &c, const float *d_inp
   k.unroll = L.g.unroll;
   k.win_floats = L.g.win;
   k.nontemporal = 1;
+  k.vec_store = (z.out_pitch % 4 == 0) && aligned16(d_output);
   k.table = plan->shifts.ptr;
   k.first_dm = o.first_dm;
   k.dm_step = o.dm_step;
@@ -746,6 +777,7 @@ dd_status prepare_step_one_f32(dd_plan *plan, const dd_conf &c, const float *d_i
   k.unroll = L.g.unroll;
   k.win_floats = L.g.win;
   k.nontemporal = 0;  // step two re-reads the intermediate
+  k.vec_store = (z.sub_out_pitch % 4 == 0) && aligned16(d_intermediate);
   k.table = plan->relative.ptr;
   k.first_dm = o.first_dm_subbanding;
   k.dm_step = o.dm_step_subbanding;
@@ -919,7 +951,7 @@ dd_status dd_plan_create(dd_plan **out, const dd_observation *obs_in, uint32_t p
     e = p->map_two.upload(m2);
     if (e != hipSuccess) return cleanup(hip_fail(e, "uploading beam mapping"));
   }
-  for (int m = 0; m < 3; ++m) p->conf[m] = default_conf((dd_mode)m);
+  set_default_confs(p);
   *out = p;
   return DD_OK;
 }
@@ -930,6 +962,7 @@ dd_status dd_plan_set_input_bits(dd_plan *plan, uint32_t input_bits) {
     return fail(DD_ERR_INVALID_ARGUMENT, "input_bits must be 1, 2, 4, 8 or 32 (float)");
   plan->input_bits = input_bits;
   size_inputs(plan);
+  set_default_confs(plan);
   return DD_OK;
 }
 
@@ -939,7 +972,9 @@ dd_status dd_plan_set_step_one_shifts(dd_plan *plan, dd_step_one_shifts delays) 
     return fail(DD_ERR_INVALID_ARGUMENT, "step-one delays must be DD_STEP_ONE_RELATIVE or DD_STEP_ONE_ABSOLUTE");
   if (!plan->two_step) return fail(DD_ERR_INVALID_ARGUMENT, "plan has no subband path");
   plan->step_one_absolute = delays == DD_STEP_ONE_ABSOLUTE;
-  return rebuild_integer_tables(plan);
+  const dd_status s = rebuild_integer_tables(plan);
+  if (s == DD_OK) set_default_confs(plan);
+  return s;
 }
 
 dd_status dd_plan_destroy(dd_plan *plan) {
@@ -960,6 +995,7 @@ dd_status dd_plan_set_conf(dd_plan *plan, dd_mode mode, const dd_conf *conf) {
   dd_status s = geometry_of(plan, mode, *conf, g);
   if (s != DD_OK) return s;
   plan->conf[mode] = *conf;
+  plan->conf_set[mode] = true;
   return DD_OK;
 }
 
@@ -1016,7 +1052,9 @@ dd_status dd_plan_set_shifts(dd_plan *plan, const float *shifts, const float *sh
     plan->h_shifts2.assign(shifts_step_two, shifts_step_two + plan->h_shifts2.size());
     DD_HIP(plan->shifts2.upload(plan->h_shifts2));
   }
-  return rebuild_integer_tables(plan);
+  const dd_status s = rebuild_integer_tables(plan);
+  if (s == DD_OK) set_default_confs(plan);
+  return s;
 }
 
 dd_status dd_plan_get_shifts(const dd_plan *plan, float *shifts, float *shifts_step_two) {

@@ -121,6 +121,7 @@ struct dd_plan {
   uint32_t input_bits = 8;  // the reference's inputBits: 1, 2, 4 (packed rows), 8, or 32 (float rows)
   dd_sizes sizes{};
   dd_conf conf[3]{};
+  bool conf_set[3]{};  // a caller's configuration (dd_plan_set_conf); else that of the plan's sizes
 
   ddamd::DeviceBuffer<float> shifts, shifts2, relative;
   std::vector<float> h_shifts, h_shifts2;
@@ -152,6 +153,8 @@ dd_status hip_fail(hipError_t e, const char *what);
 
 // Geometry of a mode under a configuration; validates limits.
 dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry &g);
+// Sets the configurations that no caller has set from the plan's sizes.
+void set_default_confs(dd_plan *p);
 // Which form of the staged byte kernel a launch takes: by the plan's own rule,
 // or one form for every job of a batch.
 enum class ByteKernel { kByRule, kVector, kMatrix };
