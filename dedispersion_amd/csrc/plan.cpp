@@ -427,22 +427,73 @@ dd_conf conf_of(uint32_t wavefronts, uint32_t items_d0, uint32_t items_d1, uint3
   return c;
 }
 
-// Step two's shape for a plan's sizes, for a plan without a caller's configuration.
-// Measured on MI355X over 32 subbands, 8-128 coarse and 16-32 fine DMs and
-// 4000-32768 samples.
-dd_conf step_two_conf(const dd_plan *p) {
+// Eight wavefronts' tile shapes, the largest first, for rows summed in one long
+// pass (the single step, and step one over 64 channels or more per subband).
+// `per_row` is the time of one row of a tile (us, in a launch of at most one
+// workgroup per compute unit), `again` that of each further such round relative
+// to the first (workgroups share a compute unit's time where two fit on it).
+// Measured at 0.2 pc/cc over 128-1536 rows, 64-2048 DMs and 2048-24576 samples:
+// the shape of least per_row x rounds is the fastest of all shapes, or within 4%
+// of it.
+struct Shape {
+  uint32_t items_d0, items_d1;
+  float per_row, again;
+};
+constexpr Shape kByteShapes[] = {{16, 8, 0.247f, 1.0f}, {8, 8, 0.193f, 1.0f}, {8, 4, 0.142f, 0.75f},
+                                 {4, 4, 0.123f, 0.66f}, {4, 2, 0.115f, 0.6f}};
+constexpr Shape kFloatShapes[] = {{16, 8, 0.77f, 1.0f}, {8, 8, 0.453f, 0.9f}, {8, 4, 0.3f, 0.88f},
+                                  {4, 4, 0.219f, 0.85f}, {4, 2, 0.15f, 0.8f}};
+
+dd_conf best_shape(const Shape (&shapes)[5], bool floats, uint32_t samples, uint32_t dms, uint64_t slices, uint32_t cus) {
+  dd_conf best{};
+  float least = 0.0f;
+  for (const Shape &h : shapes) {
+    const uint64_t nx = (samples + 64 * h.items_d0 - 1) / (64 * h.items_d0), ny = (dms + 8 * h.items_d1 - 1) / (8 * h.items_d1);
+    const uint64_t rounds = (nx * ny * slices + cus - 1) / cus;
+    const float t = h.per_row * (rounds == 1 ? 1.0f : h.again * (float)rounds);
+    if (best.unroll != 0 && t >= least) continue;
+    least = t;
+    // float rows take four copies of LDS: where rounds follow each other, fewer
+    // rows per barrier let more workgroups share a compute unit
+    best = conf_of(8, h.items_d0, h.items_d1, floats && rounds > 1 ? (h.items_d0 == 16 ? 4 : 2) : 16);
+  }
+  return best;
+}
+
+// The shape that suits a plan's sizes, for a mode without a caller's
+// configuration.  Beside the rule above, measured on MI355X over 32 subbands of
+// 8-48 channels, 8-128 coarse and 16-32 fine DMs and 4000-32768 samples.
+dd_conf default_conf(const dd_plan *p, dd_mode mode) {
   const dd_observation &o = p->obs;
   const dd_sizes &z = p->sizes;
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device);
-  // few rows (subbands) and much output: small groups of rows and many
-  // workgroups per compute unit, once there are several for each
-  const uint32_t d1 = o.nr_dms <= 16 ? 2 : o.nr_dms <= 32 ? 4 : 8;
-  const uint64_t tiles = (uint64_t)((z.nr_samples + 511) / 512) * ((o.nr_dms + 8 * d1 - 1) / (8 * d1)) *
-                         o.nr_synthesized_beams * o.nr_dms_subbanding;
-  if (tiles >= 10ull * cus && d1 == 4) return conf_of(8, 16, 4, 2);
-  if (tiles >= 4ull * cus) return conf_of(8, 8, d1, 2);
-  return conf_of(8, tiles >= (uint64_t)cus * 3 / 4 ? 8 : 4, d1, 8);
+  const bool floats = p->input_bits == 32;
+  if (mode == DD_STEP_TWO) {
+    // few rows (subbands) and much output: small groups of rows and many
+    // workgroups per compute unit, once there are several for each
+    const uint32_t d1 = o.nr_dms <= 16 ? 2 : o.nr_dms <= 32 ? 4 : 8;
+    const uint64_t tiles = (uint64_t)((z.nr_samples + 511) / 512) * ((o.nr_dms + 8 * d1 - 1) / (8 * d1)) *
+                           o.nr_synthesized_beams * o.nr_dms_subbanding;
+    if (tiles >= 10ull * cus && d1 == 4) return conf_of(8, 16, 4, 2);
+    if (tiles >= 4ull * cus) return conf_of(8, 8, d1, 2);
+    return conf_of(8, tiles >= (uint64_t)cus * 3 / 4 ? 8 : 4, d1, 8);
+  }
+  const bool single = mode == DD_SINGLE_STEP;
+  const uint32_t rows = single ? o.nr_channels : cps(p), dms = single ? o.nr_dms : o.nr_dms_subbanding;
+  const uint32_t samples = single ? z.nr_samples : z.nr_samples_step_one;
+  const uint64_t slices = single ? o.nr_synthesized_beams : (uint64_t)o.nr_beams * o.nr_subbands;
+  if (single || rows >= 64) {
+    dd_conf c = floats ? best_shape(kFloatShapes, true, samples, dms, slices, cus)
+                       : best_shape(kByteShapes, false, samples, dms, slices, cus);
+    // the vector form keeps four copies of a byte row
+    const ShiftTable &t = single ? p->ish_single : p->ish_one;
+    if (!floats && c.items_d1 >= 4 && !matrix_is_faster(rows, c.items_d1, t.mean_windows(c.items_d1)))
+      c.unroll = c.items_d0 == 16 ? 4 : c.items_d0 == 8 ? 8 : 16;
+    return c;
+  }
+  if (floats) return dms > 32 ? conf_of(8, 8, 8, 2) : dms > 16 ? conf_of(8, 8, 4, 2) : conf_of(8, 8, 2, 4);
+  return dms > 64 ? conf_of(8, 16, 8, 4) : dms > 16 ? conf_of(8, 8, 4, 8) : conf_of(8, 8, 2, 8);
 }
 
 // The shapes that every plan started from.  What they refuse (row windows too
@@ -450,7 +501,7 @@ dd_conf step_two_conf(const dd_plan *p) {
 // the shape of its sizes runs them.
 dd_conf plain_conf(dd_mode mode) {
   switch (mode) {
-  case DD_SINGLE_STEP: return conf_of(8, 16, 8, 16);
+  case DD_SINGLE_STEP: return conf_of(8, 16, 8, 4);
   case DD_STEP_ONE: return conf_of(4, 16, 8, 4);
   default: return conf_of(8, 8, 4, 8);
   }
@@ -465,8 +516,7 @@ void set_default_confs(dd_plan *p) {
     p->conf[m] = plain_conf(mode);
     if (mode != DD_SINGLE_STEP && !p->two_step) continue;
     Geometry plain, g;
-    if (mode != DD_STEP_TWO) continue;
-    const dd_conf c = step_two_conf(p);
+    const dd_conf c = default_conf(p, mode);
     if (geometry_of(p, mode, c, g) != DD_OK) continue;
     const bool packed = mode != DD_STEP_TWO && p->input_bits < 8;
     if ((g.staged && !packed) || (geometry_of(p, mode, p->conf[m], plain) == DD_OK && g.staged >= plain.staged))
