@@ -125,16 +125,16 @@ struct dd_batch {
 namespace {
 
 dd_conf batch_default_conf(dd_mode mode) {
-  // The fastest staged shape of an exhaustive sweep of both kernel kinds over
+  // The fastest staged shapes of an exhaustive sweep of both kernel kinds over
   // 40 uneven 1536-channel beams on MI355X.
   dd_conf c{};
   c.threads_d0 = 64;
   c.split_batches = 0;
   c.local = 1;
-  c.threads_d1 = 4;
-  c.items_d0 = 16;
-  c.items_d1 = 8;
-  c.unroll = 8;
+  c.threads_d1 = mode == DD_STEP_TWO ? 8 : 4;
+  c.items_d0 = mode == DD_STEP_TWO ? 8 : 16;
+  c.items_d1 = mode == DD_STEP_TWO ? 4 : 8;
+  c.unroll = mode == DD_STEP_TWO ? 4 : 8;
   return c;
 }
 
@@ -165,7 +165,7 @@ template <typename L> void merge_geometry(KindQueue &k, const L &launch, bool fi
 // sorted into the kind queues or beside them; `pairs`: prepare the compact
 // step two's paired kernel where a job allows it; `single`, `one`: the form
 // of the byte kernel of the single-step and step-one jobs.
-dd_status plan_jobs(dd_batch *b, bool pairs, ByteKernel single, ByteKernel one) {
+dd_status plan_jobs(dd_batch *b, bool pairs, bool whole, ByteKernel single, ByteKernel one) {
   for (auto &k : b->q) {
     k.u8.clear();
     k.f32.clear();
@@ -236,7 +236,7 @@ dd_status plan_jobs(dd_batch *b, bool pairs, ByteKernel single, ByteKernel one) 
         // the configuration is staged and its float form prepared: what fails
         // here is the uint16 row window or its LDS
         s = prepare_step_two_u16(job.plan, b->conf[DD_STEP_TWO], job.mid, job.out, job.first_sbeam, job.nr_sbeams,
-                                 L2, pairs);
+                                 L2, pairs, whole);
         if (s == DD_ERR_CONFIGURATION) fits = false;
         else if (s != DD_OK) return s;
       } else if (fits) {
@@ -270,6 +270,22 @@ ByteKernel common_byte_kernel(const KindQueue &k) {
   return tiles[1] >= tiles[0] ? ByteKernel::kMatrix : ByteKernel::kVector;
 }
 
+// Joins sample tiles of the uint16 step two into runs that one workgroup sums one
+// after another, while that leaves some 16 runs per compute unit (two workgroups are
+// resident on each: 8 runs one after another, of which the last may be half empty).
+void run_tiles(KindQueue &k, uint32_t cus) {
+  uint64_t tiles = 0;
+  for (const F32Launch &L : k.f32) tiles += L.k.n_tiles;
+  const uint32_t run = (uint32_t)std::min<uint64_t>(8, std::max<uint64_t>(1, tiles / (16 * cus)));
+  for (F32Launch &L : k.f32) {
+    const uint32_t others = L.k.n_tiles / L.k.n_tiles_x;
+    L.k.tiles_per_run = run;
+    L.k.n_tiles_x = (L.k.n_tiles_x + run - 1) / run;
+    L.k.n_tiles = L.k.n_tiles_x * others;
+    L.grid.x = L.k.n_tiles_x;
+  }
+}
+
 // The host part of build(): every job's launches, the per-kind geometry,
 // occupancy and tile lists (tiles[m] for kind m); no device memory is
 // touched.
@@ -299,13 +315,17 @@ dd_status plan_batch(dd_batch *b, std::vector<TileDesc> (&tiles_of)[3]) {
   // one step-two kernel for the whole batch: the paired one only when every
   // job in the batch kernels took it
   const bool pairs = b->compact && b->paired_requested;
-  dd_status st = plan_jobs(b, pairs, ByteKernel::kByRule, ByteKernel::kByRule);
+  dd_status st = plan_jobs(b, pairs, true, ByteKernel::kByRule, ByteKernel::kByRule);
   if (st != DD_OK) return st;
   bool all = true;
-  for (const F32Launch &L : b->q[DD_STEP_TWO].f32) all = all && L.g.pairs;
+  bool whole = true;  // likewise
+  for (const F32Launch &L : b->q[DD_STEP_TWO].f32) {
+    all = all && L.g.pairs;
+    whole = whole && L.g.whole;
+  }
   ByteKernel single = common_byte_kernel(b->q[DD_SINGLE_STEP]), one = common_byte_kernel(b->q[DD_STEP_ONE]);
-  if ((pairs && !all) || single != ByteKernel::kByRule || one != ByteKernel::kByRule) {
-    st = plan_jobs(b, pairs && all, single, one);
+  if ((pairs && !all) || (b->compact && !pairs && !whole) || single != ByteKernel::kByRule || one != ByteKernel::kByRule) {
+    st = plan_jobs(b, pairs && all, whole, single, one);
     if (st != DD_OK) return st;
   }
   // a job that the matrix form has no room for (its row window) takes the others with it
@@ -314,9 +334,10 @@ dd_status plan_batch(dd_batch *b, std::vector<TileDesc> (&tiles_of)[3]) {
   if (mixed_single || mixed_one) {
     if (mixed_single) single = ByteKernel::kVector;
     if (mixed_one) one = ByteKernel::kVector;
-    st = plan_jobs(b, pairs && all, single, one);
+    st = plan_jobs(b, pairs && all, whole, single, one);
     if (st != DD_OK) return st;
   }
+  if (b->compact && b->q[DD_STEP_TWO].g.whole) run_tiles(b->q[DD_STEP_TWO], (uint32_t)b->cus);
   for (int m = 0; m < 3; ++m) {
     KindQueue &k = b->q[m];
     std::vector<TileDesc> &tiles = tiles_of[m];
@@ -335,6 +356,7 @@ dd_status plan_batch(dd_batch *b, std::vector<TileDesc> (&tiles_of)[3]) {
     int per_cu = 0;
     if (m == DD_STEP_TWO) {
       if (b->compact && k.g.pairs) DD_HIP(rowsum_u16_pairs_batch_occupancy(k.g, &per_cu));
+      else if (b->compact && k.g.whole) DD_HIP(rowsum_u16_whole_batch_occupancy(k.g, &per_cu));
       else if (b->compact) DD_HIP(rowsum_u16_batch_occupancy(k.g, &per_cu));
       else DD_HIP(rowsum_f32_batch_occupancy(k.g, &per_cu));
     } else {
@@ -412,13 +434,15 @@ dd_status build(dd_batch *b) {
 // when the geometry says so.
 hipError_t launch_u16_batch(const RowSumF32Params *d_jobs, const TileQueues &tq, const Geometry &g,
                             uint32_t workgroups, hipStream_t s) {
-  return g.pairs ? launch_rowsum_u16_pairs_batch(d_jobs, tq, g, workgroups, s)
-                 : launch_rowsum_u16_batch(d_jobs, tq, g, workgroups, s);
+  return g.pairs   ? launch_rowsum_u16_pairs_batch(d_jobs, tq, g, workgroups, s)
+         : g.whole ? launch_rowsum_u16_whole_batch(d_jobs, tq, g, workgroups, s)
+                   : launch_rowsum_u16_batch(d_jobs, tq, g, workgroups, s);
 }
 hipError_t launch_u16_list(const RowSumF32Params *d_jobs, const TileDesc *d_tiles, uint32_t n, const Geometry &g,
                            hipStream_t s) {
-  return g.pairs ? launch_rowsum_u16_pairs_list(d_jobs, d_tiles, n, g, s)
-                 : launch_rowsum_u16_list(d_jobs, d_tiles, n, g, s);
+  return g.pairs   ? launch_rowsum_u16_pairs_list(d_jobs, d_tiles, n, g, s)
+         : g.whole ? launch_rowsum_u16_whole_list(d_jobs, d_tiles, n, g, s)
+                   : launch_rowsum_u16_list(d_jobs, d_tiles, n, g, s);
 }
 
 // The ordinary launches of kind m of the jobs that run beside the batch.

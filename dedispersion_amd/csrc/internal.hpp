@@ -130,6 +130,11 @@ struct RowSumF32Params {
   // difference of the pair takes over any DM tile); `unroll` then counts
   // pairs per barrier and `combine_rows` pairs added as 16-bit lanes.
   uint32_t pair_slots;
+  // Uint16 rows whole in LDS (kernels_u16_whole.hip): DMs per tile, sample tiles per
+  // run (n_tiles_x counts runs), and 2^32 / (16-byte chunks per window), rounded up.
+  uint32_t tile_dms;
+  uint32_t tiles_per_run;
+  uint32_t chunk_magic;
 };
 
 // Most LDS windows per pair of subbands in the paired step two.
@@ -149,6 +154,7 @@ struct Geometry {
   uint32_t pairs;      // 1 = the paired uint16 step two (kernels_u16_pairs.hip)
   uint32_t matrix;     // 1 = the matrix-core form of the staged kernel (kernels_u8_matrix.hip)
   uint32_t wide;       // 1 = ... whose rows may take more than one window
+  uint32_t whole;      // 1 = the uint16 step two with a tile's rows whole in LDS (kernels_u16_whole.hip)
   uint32_t many;       // 1 = the staged float kernel for slices of more than kF32Rows rows
 };
 
@@ -210,6 +216,12 @@ hipError_t launch_rowsum_u16_staged(const RowSumF32Params &p, const Geometry &g,
 hipError_t launch_rowsum_u16_batch(const RowSumF32Params *d_jobs, const TileQueues &q, const Geometry &g,
                                    uint32_t workgroups, hipStream_t stream);
 hipError_t rowsum_u16_batch_occupancy(const Geometry &g, int *per_cu);
+// The same step two with all rows of a tile in LDS at once (kernels_u16_whole.hip).
+hipError_t launch_rowsum_u16_whole_batch(const RowSumF32Params *d_jobs, const TileQueues &q, const Geometry &g,
+                                         uint32_t workgroups, hipStream_t stream);
+hipError_t launch_rowsum_u16_whole_list(const RowSumF32Params *d_jobs, const TileDesc *d_tiles, uint32_t n,
+                                        const Geometry &g, hipStream_t stream);
+hipError_t rowsum_u16_whole_batch_occupancy(const Geometry &g, int *per_cu);
 // The same step two with subbands added in pairs first (kernels_u16_pairs.hip;
 // RowSumF32Params::pair_slots set by prepare_step_two_u16).
 hipError_t launch_rowsum_u16_pairs_batch(const RowSumF32Params *d_jobs, const TileQueues &q, const Geometry &g,

@@ -252,6 +252,7 @@ dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry
   g.matrix = 0;
   g.wide = 0;
   g.many = 0;
+  g.whole = 0;
   g.unroll = c.unroll;
   // rows of floats: step two, and the single step and step one over float input
   const bool float_rows = mode == DD_STEP_TWO || p->input_bits == 32;
@@ -691,7 +692,7 @@ dd_status prepare_step_two(dd_plan *plan, const dd_conf &c, const float *d_inter
 }
 
 dd_status prepare_step_two_u16(dd_plan *plan, const dd_conf &c, const void *d_intermediate, float *d_output,
-                               uint32_t first_sbeam, uint32_t nr_sbeams, F32Launch &L, bool pairs) {
+                               uint32_t first_sbeam, uint32_t nr_sbeams, F32Launch &L, bool pairs, bool whole) {
   dd_status s = prepare_step_two(plan, c, reinterpret_cast<const float *>(d_intermediate), d_output, first_sbeam,
                                  nr_sbeams, L);
   if (s != DD_OK) return s;
@@ -719,6 +720,18 @@ dd_status prepare_step_two_u16(dd_plan *plan, const dd_conf &c, const void *d_in
   L.k.combine_rows = 65535u / bound >= 4 ? 4 : 65535u / bound >= 2 ? 2 : 1;
   L.k.pair_slots = 0;
   L.g.pairs = 0;
+  // All rows of a tile in LDS, where two workgroups per compute unit have room: one
+  // alone has nothing to sum while it stages (16 beams of 1536 channels: 0.805 ms in
+  // 512-sample tiles, two workgroups; the general kernel 0.884).  LDS: windows
+  // [rows][2 copies][win / 2 dwords] | rows | DM addresses, beside the claim slots
+  const uint64_t lds_whole = 4 * ((uint64_t)plan->obs.nr_subbands * (win + 4 + tile));
+  if (whole && !pairs && lds_whole + 16 <= plan->max_lds / 2) {
+    L.g.whole = 1;
+    L.g.lds_bytes = (uint32_t)lds_whole;
+    L.k.tile_dms = tile;
+    L.k.tiles_per_run = 1;
+    L.k.chunk_magic = (uint32_t)(0x100000000ull / (win / 8)) + 1;
+  }
   if (!pairs || 2 * bound > 65535u) return DD_OK;
   // the paired kernel: windows [2 buffers][pairs][slots][2 copies][win / 2
   // dwords]; pairs per barrier at most the wavefronts (one staging wavefront

@@ -192,9 +192,10 @@ dd_status prepare_step_two(dd_plan *plan, const dd_conf &c, const float *d_inter
 // paired kernel (kernels_u16_pairs.hip) is prepared when the job allows it
 // (a pair's sum below 2^16, at most kPairSlotsMax shift differences per pair
 // and DM tile, rows 8-element aligned, the windows within LDS); L.g.pairs
-// says which was prepared.
+// says which was prepared.  With `whole`, and not `pairs`, the kernel that keeps all
+// rows of a tile in LDS (kernels_u16_whole.hip) is prepared when they fit (L.g.whole).
 dd_status prepare_step_two_u16(dd_plan *plan, const dd_conf &c, const void *d_intermediate, float *d_output,
-                               uint32_t first_sbeam, uint32_t nr_sbeams, F32Launch &L, bool pairs = false);
+                               uint32_t first_sbeam, uint32_t nr_sbeams, F32Launch &L, bool pairs, bool whole);
 // The single step and step one over float input rows (a plan with
 // input_bits 32): the float row-sum kernels over the live-channel lists.
 dd_status prepare_single_f32(dd_plan *plan, const dd_conf &c, const float *d_input, float *d_output,
