@@ -40,9 +40,8 @@ namespace {
 // and 45, 64 rows 53 and 56, 256 rows 144 and 175, 512 rows 264 and 399; 512
 // DMs, 256 rows: 1.4 windows 102 and 101, 2.0 windows 119 and 115; 1536 rows: 1.1
 // windows 444 and 632, 1.4 windows 543 and 633, 2.0 windows 657 and 635.
-bool matrix_is_faster(uint32_t rows, uint32_t dms, float windows) {
-  if (rows < 64) return false;
-  return windows <= (dms < 8 ? 1.1f : rows > 257 ? 1.6f : 1.25f);
+bool matrix_is_faster(uint32_t rows, uint32_t dms, const ShiftTable &t) {
+  return rows >= 64 && t.mean_windows(dms) <= (dms < 8 ? 1.1f : rows > 257 ? 1.6f : 1.25f);
 }
 
 uint32_t cps(const dd_plan *p) { return p->obs.nr_channels / p->obs.nr_subbands; }
@@ -406,7 +405,7 @@ void set_byte_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, ByteKerne
   };
   const bool shaped = (c.items_d1 == 4 || c.items_d1 == 8) && g.win <= kU8MatrixWindow && lds_of(1, true) <= p->max_lds;
   g.matrix = shaped && (kernel == ByteKernel::kMatrix ||
-                        (kernel == ByteKernel::kByRule && matrix_is_faster(slots, c.items_d1, t.mean_windows(c.items_d1))));
+                        (kernel == ByteKernel::kByRule && matrix_is_faster(slots, c.items_d1, t)));
   // one window takes the first DM's shift modulo 8, the spread and the block's 8 samples
   g.wide = g.matrix && t.max_spread(c.items_d1) + 7 + 7 >= 32;
   uint32_t unroll = std::min(c.unroll, kStagedSlotsPerWave * c.threads_d1);
@@ -472,11 +471,14 @@ dd_conf default_conf(const dd_plan *p, dd_mode mode) {
   const bool floats = p->input_bits == 32;
   if (mode == DD_STEP_TWO) {
     // few rows (subbands) and much output: small groups of rows and many
-    // workgroups per compute unit, once there are several for each
+    // workgroups per compute unit, once there are several for each (both steps, us,
+    // at 16, 32, 64 and 128 coarse x 32 fine DMs and 256, 768, 3072 and 8192 tiles of
+    // 512 samples x 32 DMs: four wavefronts of 8 DMs and 2 rows per barrier 43, 60.5,
+    // 202 and 478; eight wavefronts of 4 DMs and 8 rows 36.5, 69, 245 and 619)
     const uint32_t d1 = o.nr_dms <= 16 ? 2 : o.nr_dms <= 32 ? 4 : 8;
     const uint64_t tiles = (uint64_t)((z.nr_samples + 511) / 512) * ((o.nr_dms + 8 * d1 - 1) / (8 * d1)) *
                            o.nr_synthesized_beams * o.nr_dms_subbanding;
-    if (tiles >= 10ull * cus && d1 == 4) return conf_of(8, 16, 4, 2);
+    if (tiles >= 2ull * cus && d1 == 4) return conf_of(4, 8, 8, 2);
     if (tiles >= 4ull * cus) return conf_of(8, 8, d1, 2);
     return conf_of(8, tiles >= (uint64_t)cus * 3 / 4 ? 8 : 4, d1, 8);
   }
@@ -489,7 +491,7 @@ dd_conf default_conf(const dd_plan *p, dd_mode mode) {
                        : best_shape(kByteShapes, false, samples, dms, slices, cus);
     // the vector form keeps four copies of a byte row
     const ShiftTable &t = single ? p->ish_single : p->ish_one;
-    if (!floats && c.items_d1 >= 4 && !matrix_is_faster(rows, c.items_d1, t.mean_windows(c.items_d1)))
+    if (!floats && c.items_d1 >= 4 && !matrix_is_faster(rows, c.items_d1, t))
       c.unroll = c.items_d0 == 16 ? 4 : c.items_d0 == 8 ? 8 : 16;
     return c;
   }
