@@ -236,6 +236,28 @@ dd_status build_factored(dd_plan *p) {
 
 } // namespace
 
+namespace {
+
+uint32_t compute_units(const dd_plan *p) {
+  int n = 256;
+  (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, p->device);
+  return (uint32_t)n;
+}
+
+// Workgroups of a launch over float rows, all beams.
+uint64_t float_tiles(const dd_plan *p, dd_mode mode, uint32_t samples_per_tile, uint32_t dms_per_tile) {
+  const dd_observation &o = p->obs;
+  const dd_sizes &z = p->sizes;
+  const uint32_t samples = mode == DD_STEP_ONE ? z.nr_samples_step_one : z.nr_samples;
+  const uint32_t dms = mode == DD_STEP_ONE ? o.nr_dms_subbanding : o.nr_dms;
+  const uint64_t slices = mode == DD_SINGLE_STEP ? o.nr_synthesized_beams
+                          : mode == DD_STEP_ONE  ? (uint64_t)o.nr_beams * o.nr_subbands
+                                                 : (uint64_t)o.nr_synthesized_beams * o.nr_dms_subbanding;
+  return (uint64_t)((samples + samples_per_tile - 1) / samples_per_tile) * ((dms + dms_per_tile - 1) / dms_per_tile) * slices;
+}
+
+} // namespace
+
 dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry &g) {
   if (c.split_batches) return fail(DD_ERR_UNSUPPORTED, "split batches mode is not implemented");
   if (c.threads_d0 != 64) return fail(DD_ERR_CONFIGURATION, "threads_d0 must be 64 (one wavefront along samples)");
@@ -330,8 +352,15 @@ dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry
         const uint32_t slots = mode == DD_STEP_TWO ? p->obs.nr_subbands
                                : mode == DD_SINGLE_STEP ? p->obs.nr_channels : cps(p);
         auto lds_of = [&](uint32_t u) { return 4 * (4 * std::min(slots, kF32Rows) + 8 * u * g.win + 2 * u * tile); };
+        // A grid of more than one workgroup per compute unit leaves room for 16
+        // wavefronts on each, which the registers of all but the largest shapes
+        // allow (step two of 64 x 32 DMs x 24576 samples, eight wavefronts of 4 DMs:
+        // 8 rows per barrier and one workgroup 157 us, 4 rows and two 116).
+        const uint64_t tiles = float_tiles(p, mode, ts, tile);
+        const bool share = tiles > compute_units(p) && c.items_d0 * c.items_d1 <= 64;
+        const uint64_t room = share ? std::min<uint64_t>(p->max_lds, (uint64_t)p->max_lds * c.threads_d1 / 16) : p->max_lds;
         uint32_t unroll = c.unroll;
-        while (unroll > 1 && lds_of(unroll) > p->max_lds) --unroll;
+        while (unroll > 1 && lds_of(unroll) > room) --unroll;
         if (lds_of(unroll) <= p->max_lds) {
           g.staged = 1;
           g.many = slots > kF32Rows;
@@ -466,8 +495,7 @@ dd_conf best_shape(const Shape (&shapes)[5], bool floats, uint32_t samples, uint
 dd_conf default_conf(const dd_plan *p, dd_mode mode) {
   const dd_observation &o = p->obs;
   const dd_sizes &z = p->sizes;
-  int cus = 256;
-  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device);
+  const uint32_t cus = compute_units(p);
   const bool floats = p->input_bits == 32;
   if (mode == DD_STEP_TWO) {
     // few rows (subbands) and much output: small groups of rows and many
