@@ -210,8 +210,8 @@ hipError_t launch_rowsum_u16_list(const RowSumF32Params *d_jobs, const TileDesc 
 hipError_t rowsum_f32_batch_occupancy(const Geometry &g, int *per_cu);
 hipError_t launch_clear_words(uint32_t *d_words, uint32_t n, hipStream_t stream);
 // Step two over uint16 step-one sums (kernels_u16_staged.hip): the staged
-// pipeline with a window of g.win uint16 elements per row, two copies per
-// row (shifted by one element) so that every read is dword aligned.
+// pipeline with a window of g.win uint16 elements per row, four copies per
+// row (shifted by an element each) so that every read is 8-byte aligned.
 hipError_t launch_rowsum_u16_staged(const RowSumF32Params &p, const Geometry &g, hipStream_t stream);
 hipError_t launch_rowsum_u16_batch(const RowSumF32Params *d_jobs, const TileQueues &q, const Geometry &g,
                                    uint32_t workgroups, hipStream_t stream);

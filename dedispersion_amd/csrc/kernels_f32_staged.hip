@@ -24,7 +24,7 @@
 // 12288 samples 1648 -> 538, best 381 -> 328; 256 x 2048 x 24576 best 690 -> 586
 // (22e12 additions per second); step one, 32 channels x 32 coarse DMs x 20000
 // samples x 32 subbands, best 64.2 -> 51.6; step two, 32 subbands x 2048 DMs x
-// 20000, 124 -> 115 (72% of it the output's 164 MB at the rate of a fill).
+// 24576, 124 -> 114 (its loads and stores alone take 100, its sums 73).
 #include "staged_common.hpp"
 
 namespace ddamd {
@@ -36,7 +36,7 @@ using namespace staged;
 // the launch described by p (DM tile fastest).
 // MANY: a slice may have more rows than kF32Rows, and they are listed in LDS that
 // many at a time (a loop that costs 5-10 registers: a wavefront per SIMD at RUN 8 and
-// 4 DMs, 231 against 201 us over both steps of 1536 channels x 2048 DMs x 20000).
+// 4 DMs, 231 against 201 us over both steps of 1536 channels x 2048 DMs x 24576).
 template <int RUN, int DPW, bool MANY>
 __device__ __forceinline__ void f32_tile(const RowSumF32Params &p, uint32_t logical, float *ldsf) {
   constexpr int TS = 64 * RUN;
