@@ -32,7 +32,7 @@ dd_status hip_fail(hipError_t e, const char *what) {
 namespace {
 
 // Whether the matrix-core byte kernel sums `rows` rows faster than the vector
-// one, with `dms` DMs per wavefront and `windows` windows per row on average:
+// one, with `dms` DMs per wavefront, by the windows per row on average:
 // its products grow with the windows, the vector kernel's additions do not;
 // eight DMs share the operands that four read; above 257 rows the vector kernel
 // spills its 16-bit sums to 32 bits.  Measured (us, matrix against vector form,
@@ -238,12 +238,6 @@ dd_status build_factored(dd_plan *p) {
 
 namespace {
 
-uint32_t compute_units(const dd_plan *p) {
-  int n = 256;
-  (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, p->device);
-  return (uint32_t)n;
-}
-
 // Workgroups of a launch over float rows, all beams.
 uint64_t float_tiles(const dd_plan *p, dd_mode mode, uint32_t samples_per_tile, uint32_t dms_per_tile) {
   const dd_observation &o = p->obs;
@@ -357,7 +351,7 @@ dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry
         // allow (step two of 64 x 32 DMs x 24576 samples, eight wavefronts of 4 DMs:
         // 8 rows per barrier and one workgroup 157 us, 4 rows and two 116).
         const uint64_t tiles = float_tiles(p, mode, ts, tile);
-        const bool share = tiles > compute_units(p) && c.items_d0 * c.items_d1 <= 64;
+        const bool share = tiles > p->compute_units && c.items_d0 * c.items_d1 <= 64;
         const uint64_t room = share ? std::min<uint64_t>(p->max_lds, (uint64_t)p->max_lds * c.threads_d1 / 16) : p->max_lds;
         uint32_t unroll = c.unroll;
         while (unroll > 1 && lds_of(unroll) > room) --unroll;
@@ -495,7 +489,7 @@ dd_conf best_shape(const Shape (&shapes)[5], bool floats, uint32_t samples, uint
 dd_conf default_conf(const dd_plan *p, dd_mode mode) {
   const dd_observation &o = p->obs;
   const dd_sizes &z = p->sizes;
-  const uint32_t cus = compute_units(p);
+  const uint32_t cus = p->compute_units;
   const bool floats = p->input_bits == 32;
   if (mode == DD_STEP_TWO) {
     // few rows (subbands) and much output: small groups of rows and many
@@ -956,7 +950,10 @@ dd_status dd_plan_create(dd_plan **out, const dd_observation *obs_in, uint32_t p
   p->two_step = o.nr_dms_subbanding > 0;
   (void)hipGetDevice(&p->device);
   hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, p->device) == hipSuccess) p->max_lds = prop.sharedMemPerBlock;
+  if (hipGetDeviceProperties(&prop, p->device) == hipSuccess) {
+    p->max_lds = prop.sharedMemPerBlock;
+    p->compute_units = (uint32_t)prop.multiProcessorCount;
+  }
 
   auto cleanup = [&](dd_status s) {
     delete p;

@@ -117,6 +117,7 @@ struct dd_plan {
   uint32_t padding = 0;
   int device = 0;
   size_t max_lds = 65536;
+  uint32_t compute_units = 256;
   bool two_step = false;
   bool step_one_absolute = false;  // step one applies each channel's own delay (dd_plan_set_step_one_shifts)
   uint32_t input_bits = 8;  // the reference's inputBits: 1, 2, 4 (packed rows), 8, or 32 (float rows)
