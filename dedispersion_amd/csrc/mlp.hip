@@ -310,12 +310,13 @@ struct dd_mlp {
   size_t count = 0;
   float *params = nullptr, *m = nullptr, *v = nullptr, *grad_tmp = nullptr;
   uint32_t step = 0;
-  // parts of the gradient, one per workgroup, and the losses of a training run
-  float *part = nullptr, *losses = nullptr;
-  uint32_t part_groups = 0, losses_cap = 0;
+  // parts of the gradient, one per workgroup, the losses of a training run, and
+  // the outputs of a forward pass whose caller wants them inside its input
+  float *part = nullptr, *losses = nullptr, *outputs = nullptr;
+  uint32_t part_groups = 0, losses_cap = 0, outputs_cap = 0;
 
   ~dd_mlp() {
-    for (float *p : {params, m, v, grad_tmp, part, losses}) (void)hipFree(p);
+    for (float *p : {params, m, v, grad_tmp, part, losses, outputs}) (void)hipFree(p);
   }
 };
 
@@ -474,7 +475,16 @@ dd_status dd_mlp_init(dd_mlp *net, uint64_t seed) {
 dd_status dd_mlp_forward(dd_mlp *net, const float *d_x, uint32_t n, float *d_y, void *stream) {
   if (!net || !d_x || !d_y) return fail_mlp(DD_ERR_INVALID_ARGUMENT, "null argument");
   if (n == 0) return DD_OK;
-  return forward(net, d_x, n, d_y, (hipStream_t)stream);
+  // A workgroup stores its rows' outputs while others still read their inputs, so
+  // outputs inside the input are written once the pass is over.
+  const uintptr_t x0 = reinterpret_cast<uintptr_t>(d_x), x1 = x0 + (size_t)n * net->shape.inputs * sizeof(float);
+  const uintptr_t y0 = reinterpret_cast<uintptr_t>(d_y), y1 = y0 + (size_t)n * sizeof(float);
+  if (y1 <= x0 || x1 <= y0) return forward(net, d_x, n, d_y, (hipStream_t)stream);
+  dd_status s = reserve(net->outputs, net->outputs_cap, n, 1);
+  if (s == DD_OK) s = forward(net, d_x, n, net->outputs, (hipStream_t)stream);
+  if (s != DD_OK) return s;
+  MLP_HIP(hipMemcpyAsync(d_y, net->outputs, (size_t)n * sizeof(float), hipMemcpyDeviceToDevice, (hipStream_t)stream));
+  return DD_OK;
 }
 
 dd_status dd_mlp_loss_grad(dd_mlp *net, const float *d_x, const float *d_target, uint32_t n, float *d_loss,

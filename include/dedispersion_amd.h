@@ -509,7 +509,7 @@ dd_status dd_mlp_set_params(dd_mlp *net, const float *params); /* host array; re
 dd_status dd_mlp_get_params(const dd_mlp *net, float *params); /* host array */
 /* He-uniform weights from `seed`, zero biases. */
 dd_status dd_mlp_init(dd_mlp *net, uint64_t seed);
-/* d_y[r] = network(d_x[r][0..inputs)) for r < n. */
+/* d_y[r] = network(d_x[r][0..inputs)) for r < n; d_y may lie inside d_x. */
 dd_status dd_mlp_forward(dd_mlp *net, const float *d_x, uint32_t n, float *d_y, void *stream);
 /* Mean squared error L = (1/n) sum (y_r - t_r)^2 into d_loss[0] and dL/dparams
  * into d_grad (flat parameter layout). */

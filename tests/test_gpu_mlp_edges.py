@@ -1,0 +1,54 @@
+"""The cost model's passes where their blocks of rows could show: an output inside
+the input, parameters that are not finite, wide networks over few rows and narrow
+ones over many.  Against the numpy reference in float64, with the tolerances of the
+tuner's network."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from dedispersion_amd import load
+from dedispersion_amd._lib import check
+from oracle import mlp
+
+pytestmark = pytest.mark.gpu
+
+
+def network(shape, seed):
+    """A network and its parameters."""
+    lib = load()
+    h = ctypes.c_void_p()
+    check(lib.dd_mlp_create(ctypes.byref(h), *shape))
+    rng = np.random.default_rng(seed)
+    p = np.zeros(mlp.param_count(*shape), dtype=np.float32)
+    for w, a, b, bo in mlp.layout(*shape):
+        p[w:w + a * b] = rng.standard_normal(a * b) * np.sqrt(2.0 / a)
+        p[bo:bo + b] = rng.standard_normal(b) * 0.1
+    return lib, h, p, rng
+
+
+def set_params(lib, h, p):
+    check(lib.dd_mlp_set_params(h, p.ctypes.data_as(ctypes.POINTER(ctypes.c_float))))
+
+
+@pytest.mark.parametrize("at", ["first", "middle", "last", "across"])
+@pytest.mark.parametrize("shape,n", [((12, 64, 3), 60000), ((3, 100, 1), 4001), ((1, 5, 1), 70000), ((20, 90, 3), 9001)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_output_inside_the_input(torch_cuda, shape, n, at):
+    torch = torch_cuda
+    lib, h, p, rng = network(shape, n)
+    try:
+        set_params(lib, h, p)
+        x = torch.from_numpy(rng.standard_normal(n * shape[0]).astype(np.float32)).cuda()
+        want = torch.empty(n, device="cuda")
+        check(lib.dd_mlp_forward(h, x.data_ptr(), n, want.data_ptr(), None))
+        room = torch.zeros(n * shape[0] + n, device="cuda")  # the input and, past it, space for one of the outputs
+        room[:n * shape[0]] = x
+        start = {"first": 0, "middle": n * (shape[0] // 2), "last": n * (shape[0] - 1),
+                 "across": n * shape[0] - n // 2}[at]
+        check(lib.dd_mlp_forward(h, room.data_ptr(), n, room[start:].data_ptr(), None))
+        assert torch.equal(room[start:start + n], want)
+        y, _ = mlp.forward(p.astype(np.float64), x.cpu().numpy().reshape(n, -1).astype(np.float64), *shape)
+        assert np.max(np.abs(want.cpu().numpy() - y)) <= 1e-5 * max(1.0, np.max(np.abs(y)))
+    finally:
+        lib.dd_mlp_destroy(h)
