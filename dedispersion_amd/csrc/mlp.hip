@@ -109,15 +109,18 @@ __device__ __forceinline__ void add_products(float4 &acc, const float *e, const 
 
 // One layer over R rows held unit by unit (in[i * R + r]): out[j][r] = act(b[j]
 // + sum over i, in order, of in[i][r] W[i][j]); a thread takes four rows of a
-// unit, and consecutive threads consecutive units.
+// unit, and consecutive threads consecutive units.  Rows from `rows` on are zero.
 template <uint32_t R>
-__device__ __forceinline__ void dense(const Layer &y, uint32_t din, uint32_t dout, bool relu, const float *in, float *out) {
+__device__ __forceinline__ void dense(const Layer &y, uint32_t din, uint32_t dout, bool relu, const float *in, float *out,
+                                      uint32_t rows = R) {
   for (uint32_t idx = threadIdx.x; idx < dout * (R / 4); idx += blockDim.x) {
     const uint32_t j = idx % dout, q = 4 * (idx / dout);
     const float bias = y.b[j];
     float4 acc = make_float4(bias, bias, bias, bias);
     add_products<R>(acc, in + q, y.W + j, din, y.ld);
     if (relu) acc = make_float4(fmaxf(acc.x, 0.0f), fmaxf(acc.y, 0.0f), fmaxf(acc.z, 0.0f), fmaxf(acc.w, 0.0f));
+    if (q + 4 > rows)
+      acc = make_float4(q < rows ? acc.x : 0.0f, q + 1 < rows ? acc.y : 0.0f, q + 2 < rows ? acc.z : 0.0f, 0.0f);
     *reinterpret_cast<float4 *>(out + j * R + q) = acc;
   }
 }
@@ -181,11 +184,14 @@ __global__ void __launch_bounds__(256) mlp_gradient(const Shape s, const float *
   auto input_of = [&](uint32_t l) { return act + (l == 0 ? 0 : (s.inputs + (l - 1) * s.hidden) * R); };
   bool first = true;
   for (uint64_t r0 = (uint64_t)blockIdx.x * R; r0 < n; r0 += (uint64_t)gridDim.x * R, first = false) {
+    // rows past n stay zero in every layer: their errors are zero, and zero times
+    // an activation that is not finite would not be
+    const uint32_t rows = (uint32_t)min((uint64_t)R, n - r0);
     read_rows<R>(X, n, s.inputs, r0, act);
     __syncthreads();
     for (uint32_t l = 0; l <= s.layers; ++l) {
       dense<R>(layer_of<RESIDENT>(s, l, params, weights), s.fan_in(l), s.fan_out(l), l < s.layers, input_of(l),
-               l < s.layers ? input_of(l + 1) : GX);
+               l < s.layers ? input_of(l + 1) : GX, rows);
       __syncthreads();
     }
     // the output's error 2 (y - t) / n, and the squares

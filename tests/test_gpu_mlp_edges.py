@@ -52,3 +52,36 @@ def test_output_inside_the_input(torch_cuda, shape, n, at):
         assert np.max(np.abs(want.cpu().numpy() - y)) <= 1e-5 * max(1.0, np.max(np.abs(y)))
     finally:
         lib.dd_mlp_destroy(h)
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 35])
+@pytest.mark.parametrize("shape", [(3, 16, 1), (4, 12, 3), (5, 130, 1)], ids=lambda v: "x".join(map(str, v)))
+@pytest.mark.parametrize("where", ["bias", "weight"])
+def test_parameters_that_are_not_finite(torch_cuda, where, shape, n):
+    """A unit of the first layer that is +inf for every row: what the gradient's
+    elements are -- finite, an infinity or NaN -- is what the sums over the n rows
+    give, whatever fills a block of rows past them."""
+    torch = torch_cuda
+    lib, h, p, rng = network(shape, n)
+    try:
+        # all positive, so that no sum meets infinities of both signs
+        x = np.abs(rng.standard_normal((n, shape[0]))).astype(np.float32) + 0.5
+        t = rng.standard_normal(n).astype(np.float32)
+        p = np.abs(p) + np.float32(0.01)
+        w, a, b, bo = mlp.layout(*shape)[0]
+        if where == "bias":
+            p[bo + 2] = np.inf
+        else:
+            p[w + 2] = np.inf  # input 0 to unit 2
+        set_params(lib, h, p)
+        dx, dt = torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda()
+        dl, dg = (torch.full((k,), 7.0, dtype=torch.float32, device="cuda") for k in (1, p.size))
+        check(lib.dd_mlp_loss_grad(h, dx.data_ptr(), dt.data_ptr(), n, dl.data_ptr(), dg.data_ptr(), None))
+        with np.errstate(all="ignore"):
+            loss, want = mlp.loss_grad(p.astype(np.float64), x.astype(np.float64), t.astype(np.float64), *shape)
+        got = dg.cpu().numpy()
+        assert np.isinf(want).any() and np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(np.float32))
+        assert np.isinf(loss) and float(dl[0]) == loss
+    finally:
+        lib.dd_mlp_destroy(h)
