@@ -43,9 +43,9 @@ struct Shape {
   __host__ __device__ uint32_t lds_floats() const { return (lds_offset(layers) + 2 * hidden + 1 + 3) & ~3u; }
 };
 
-constexpr uint32_t kColumns = 16;       // columns of a weight matrix transposed through LDS at a time
+constexpr uint32_t kColumns = 32;       // columns of a weight matrix transposed through LDS at a time
 constexpr uint32_t kMaxGroups = 512;    // workgroups of the gradient pass (partial gradients)
-constexpr uint32_t kMaxLds = 64 * 1024;
+constexpr uint32_t kResidentLds = 64 * 1024;  // a workgroup's, where its weights stay in LDS: two per compute unit
 
 // A layer's weights W[i * ld + j] and biases, in LDS or in the parameter array.
 struct Layer {
@@ -157,6 +157,13 @@ __global__ void __launch_bounds__(256) mlp_forward(const Shape s, const float *_
   if (threadIdx.x < R && r0 + threadIdx.x < n) Y[r0 + threadIdx.x] = in[threadIdx.x];
 }
 
+// Threads of a workgroup of the gradient pass.  Weights that are not in LDS are
+// waited for; twice the threads have twice the reads under way (four rows of
+// 256 x 256 x 8 networks: 802 us with 256 threads, 16 columns at a time and one
+// read after another; 691 with the reads in batches; 347 with 512 threads and 32
+// columns; one launch per layer and operation took 458).
+constexpr uint32_t gradient_threads(bool resident) { return resident ? 256 : 512; }
+
 // Forward and backward pass of L = (1/n) sum_r (y_r - t_r)^2 over R rows at a
 // time.  Activations and errors stay in LDS.  Workgroup g takes row blocks g, g
 // + gridDim.x, ... and leaves its part of dL/dparams in part[g * (count + 1)],
@@ -169,7 +176,7 @@ __global__ void __launch_bounds__(256) mlp_forward(const Shape s, const float *_
 // one workgroup's chain of layers, so a workgroup takes as few rows as still
 // share a weight read.
 template <uint32_t R, bool RESIDENT>
-__global__ void __launch_bounds__(256) mlp_gradient(const Shape s, const float *__restrict__ X,
+__global__ void __launch_bounds__(gradient_threads(RESIDENT)) mlp_gradient(const Shape s, const float *__restrict__ X,
                                                     const float *__restrict__ T, uint32_t n,
                                                     const float *__restrict__ params, uint32_t count,
                                                     float *__restrict__ part) {
@@ -214,8 +221,9 @@ __global__ void __launch_bounds__(256) mlp_gradient(const Shape s, const float *
       // weights W[i][j] and, as row i = a, the biases
       uint32_t held = ~0u;
       float4 g[R / 4];
+      const uint32_t di = blockDim.x / b, dj = blockDim.x % b;
+      uint32_t i = threadIdx.x / b, j = threadIdx.x % b;
       for (uint32_t idx = threadIdx.x; idx < (a + 1) * b; idx += blockDim.x) {
-        const uint32_t i = idx / b, j = idx % b;
         if (j != held) {
           held = j;
 #pragma unroll
@@ -232,6 +240,12 @@ __global__ void __launch_bounds__(256) mlp_gradient(const Shape s, const float *
         }
         float *slot = mine + s.offset(l) + idx;
         *slot = first ? sum : *slot + sum;
+        i += di;
+        j += dj;
+        if (j >= b) {
+          j -= b;
+          ++i;
+        }
       }
       if (l == 0) break;
       // the layer input's error, through the ReLU of the layer below: GX[i][r] =
@@ -243,9 +257,19 @@ __global__ void __launch_bounds__(256) mlp_gradient(const Shape s, const float *
         const uint32_t nj = b - j0 < step ? b - j0 : step;
         if (!RESIDENT) {
           __syncthreads();
-          for (uint32_t idx = threadIdx.x; idx < a * kColumns; idx += blockDim.x) {
-            const uint32_t i = idx / kColumns, c = idx % kColumns;
-            if (c < nj) cols[i * (kColumns + 1) + c] = y.W[i * y.ld + j0 + c];
+          constexpr uint32_t kInFlight = 16;
+          for (uint32_t x0 = threadIdx.x; x0 < a * kColumns; x0 += kInFlight * blockDim.x) {
+            float v[kInFlight];
+#pragma unroll
+            for (uint32_t k = 0; k < kInFlight; ++k) {
+              const uint32_t idx = min(x0 + k * blockDim.x, a * kColumns - 1);
+              v[k] = y.W[idx / kColumns * y.ld + j0 + min(idx % kColumns, nj - 1)];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < kInFlight; ++k) {
+              const uint32_t idx = x0 + k * blockDim.x;
+              if (idx < a * kColumns) cols[idx / kColumns * (kColumns + 1) + idx % kColumns] = v[k];
+            }
           }
           __syncthreads();
         }
@@ -350,7 +374,7 @@ uint32_t forward_lds(const Shape &s, uint32_t R, bool resident) {
 
 // The weights are kept in LDS where 16 rows' activations fit beside them (up to
 // three hidden layers of 64, or one of 100); else a workgroup takes four rows.
-bool resident(const Shape &s) { return gradient_lds(s, 16, true) <= kMaxLds; }
+bool resident(const Shape &s) { return gradient_lds(s, 16, true) <= kResidentLds; }
 uint32_t gradient_rows(const Shape &s) { return resident(s) ? 16 : 4; }
 
 uint32_t gradient_groups(const Shape &s, uint32_t n) {
@@ -389,7 +413,7 @@ dd_status loss_grad(dd_mlp *net, const float *d_x, const float *d_t, uint32_t n,
   const uint32_t groups = gradient_groups(sh, n);
   const bool keep = resident(sh);
   auto kernel = keep ? mlp_gradient<16, true> : mlp_gradient<4, false>;
-  hipLaunchKernelGGL(kernel, dim3(groups), dim3(256), gradient_lds(sh, gradient_rows(sh), keep), s, sh, d_x, d_t, n,
+  hipLaunchKernelGGL(kernel, dim3(groups), dim3(gradient_threads(keep)), gradient_lds(sh, gradient_rows(sh), keep), s, sh, d_x, d_t, n,
                      net->params, (uint32_t)net->count, net->part);
   MLP_HIP(hipGetLastError());
   hipLaunchKernelGGL(mlp_sum_parts, dim3(blocks_for(net->count + 1, 64)), dim3(256), 0, s, net->part, groups,

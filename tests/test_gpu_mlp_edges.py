@@ -85,3 +85,29 @@ def test_parameters_that_are_not_finite(torch_cuda, where, shape, n):
         assert np.isinf(loss) and float(dl[0]) == loss
     finally:
         lib.dd_mlp_destroy(h)
+
+
+# networks whose weights are read a few columns at a time: widths on both sides of
+# whole blocks of columns and of a workgroup's threads, and rows of one to three blocks
+@pytest.mark.parametrize("shape,n", [((9, 95, 4), 5), ((9, 96, 4), 4), ((9, 97, 4), 3), ((2, 129, 2), 12), ((256, 255, 2), 6),
+                                     ((256, 256, 8), 9), ((33, 160, 5), 1), ((256, 200, 3), 2053)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_wide_networks(torch_cuda, shape, n):
+    torch = torch_cuda
+    lib, h, p, rng = network(shape, n)
+    try:
+        x = rng.standard_normal((n, shape[0])).astype(np.float32)
+        t = rng.standard_normal(n).astype(np.float32)
+        set_params(lib, h, p)
+        dx, dt = torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda()
+        dl, dg = (torch.full((k,), 7.0, dtype=torch.float32, device="cuda") for k in (1, p.size))
+        check(lib.dd_mlp_loss_grad(h, dx.data_ptr(), dt.data_ptr(), n, dl.data_ptr(), dg.data_ptr(), None))
+        loss, grad = mlp.loss_grad(p.astype(np.float64), x.astype(np.float64), t.astype(np.float64), *shape)
+        assert abs(float(dl[0]) - loss) <= 1e-5 * max(1.0, loss)
+        g = dg.cpu().numpy()
+        for w, a, b, bo in mlp.layout(*shape):
+            for lo, hi in ((w, w + a * b), (bo, bo + b)):
+                scale = max(np.max(np.abs(grad[lo:hi])), 1e-12)
+                assert np.max(np.abs(g[lo:hi] - grad[lo:hi])) <= 2e-4 * scale, (lo, hi)
+    finally:
+        lib.dd_mlp_destroy(h)
