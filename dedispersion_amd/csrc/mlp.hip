@@ -45,6 +45,7 @@ struct Shape {
 
 constexpr uint32_t kColumns = 32;       // columns of a weight matrix transposed through LDS at a time
 constexpr uint32_t kMaxGroups = 512;    // workgroups of the gradient pass (partial gradients)
+constexpr uint32_t kMaxParts = 1u << 27;  // floats of their partial gradients (512 MiB; 1 GiB is 1.5x faster at most)
 constexpr uint32_t kResidentLds = 64 * 1024;  // a workgroup's, where its weights stay in LDS: two per compute unit
 
 // A layer's weights W[i * ld + j] and biases, in LDS or in the parameter array.
@@ -377,8 +378,11 @@ uint32_t forward_lds(const Shape &s, uint32_t R, bool resident) {
 bool resident(const Shape &s) { return gradient_lds(s, 16, true) <= kResidentLds; }
 uint32_t gradient_rows(const Shape &s) { return resident(s) ? 16 : 4; }
 
+// The parts of all workgroups take at most kMaxParts floats, which networks of more
+// than 262143 parameters reach below kMaxGroups.
 uint32_t gradient_groups(const Shape &s, uint32_t n) {
-  return std::min(blocks_for(n, gradient_rows(s)), kMaxGroups);
+  const uint32_t count = s.offset(s.layers) + s.hidden + 1;
+  return std::min(blocks_for(n, gradient_rows(s)), std::min(kMaxGroups, kMaxParts / (count + 1)));
 }
 
 dd_status reserve(float *&p, uint32_t &have, uint32_t want, size_t each) {

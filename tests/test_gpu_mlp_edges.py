@@ -111,3 +111,20 @@ def test_wide_networks(torch_cuda, shape, n):
                 assert np.max(np.abs(g[lo:hi] - grad[lo:hi])) <= 2e-4 * scale, (lo, hi)
     finally:
         lib.dd_mlp_destroy(h)
+
+
+def test_largest_network_takes_bounded_memory(torch_cuda):
+    """The partial gradients of 256 x 256 x 8 over 2880 rows: at most 512 MiB."""
+    torch = torch_cuda
+    shape, n = (256, 256, 8), 2880
+    lib, h, p, rng = network(shape, n)
+    try:
+        set_params(lib, h, p)
+        dx, dt, dl, dg = (torch.zeros(k, dtype=torch.float32, device="cuda") for k in (n * shape[0], n, 1, p.size))
+        torch.cuda.synchronize()
+        free, _ = torch.cuda.mem_get_info()
+        check(lib.dd_mlp_loss_grad(h, dx.data_ptr(), dt.data_ptr(), n, dl.data_ptr(), dg.data_ptr(), None))
+        torch.cuda.synchronize()
+        assert free - torch.cuda.mem_get_info()[0] <= (512 << 20) + (4 << 20)  # and the allocator's granularity
+    finally:
+        lib.dd_mlp_destroy(h)
