@@ -46,7 +46,8 @@ struct Shape {
 constexpr uint32_t kColumns = 32;       // columns of a weight matrix transposed through LDS at a time
 constexpr uint32_t kMaxGroups = 512;    // workgroups of the gradient pass (partial gradients)
 constexpr uint32_t kMaxParts = 1u << 27;  // floats of their partial gradients (512 MiB; 1 GiB is 1.5x faster at most)
-constexpr uint32_t kResidentLds = 64 * 1024;  // a workgroup's, where its weights stay in LDS: two per compute unit
+constexpr uint32_t kHalfLds = 80 * 1024;      // LDS of a workgroup that shares a compute unit with another
+constexpr uint32_t kResidentLds = 64 * 1024;  // ... whose weights stay in LDS
 
 // A layer's weights W[i * ld + j] and biases, in LDS or in the parameter array.
 struct Layer {
@@ -110,8 +111,8 @@ __device__ __forceinline__ void add_products(float4 &acc, const float *e, const 
 
 // One layer over R rows held unit by unit (in[i * R + r]): out[j][r] = act(b[j]
 // + sum over i, in order, of in[i][r] W[i][j]); a thread takes four rows of a
-// unit, and consecutive threads consecutive units.  Rows from `rows` on are zero.
-template <uint32_t R>
+// unit, and consecutive threads consecutive units.  CUT: rows from `rows` on are zero.
+template <uint32_t R, bool CUT>
 __device__ __forceinline__ void dense(const Layer &y, uint32_t din, uint32_t dout, bool relu, const float *in, float *out,
                                       uint32_t rows = R) {
   for (uint32_t idx = threadIdx.x; idx < dout * (R / 4); idx += blockDim.x) {
@@ -120,18 +121,43 @@ __device__ __forceinline__ void dense(const Layer &y, uint32_t din, uint32_t dou
     float4 acc = make_float4(bias, bias, bias, bias);
     add_products<R>(acc, in + q, y.W + j, din, y.ld);
     if (relu) acc = make_float4(fmaxf(acc.x, 0.0f), fmaxf(acc.y, 0.0f), fmaxf(acc.z, 0.0f), fmaxf(acc.w, 0.0f));
-    if (q + 4 > rows)
+    if (CUT && q + 4 > rows)
       acc = make_float4(q < rows ? acc.x : 0.0f, q + 1 < rows ? acc.y : 0.0f, q + 2 < rows ? acc.z : 0.0f, 0.0f);
     *reinterpret_cast<float4 *>(out + j * R + q) = acc;
   }
 }
 
-// Rows r0 .. r0 + R - 1 of X (n x inputs) to in[i * R + r]; zeros past row n.
+// Rows r0 .. r0 + R - 1 of X (n x inputs) to in[i * R + r]; zeros past row n.  Few
+// rows are read in the order of the input.  Of 64, a thread takes four inputs of a
+// row and consecutive threads consecutive rows, whose places in LDS lie side by side
+// (in the input's order they are 64 floats apart, all on one bank: 260 against 210 us
+// for 200000 rows of 256 x 8 x 1; over 16 rows it costs 0.7 us more latency).
 template <uint32_t R>
 __device__ __forceinline__ void read_rows(const float *__restrict__ X, uint32_t n, uint32_t inputs, uint64_t r0, float *in) {
-  for (uint32_t idx = threadIdx.x; idx < inputs * R; idx += blockDim.x) {
-    const uint32_t r = idx / inputs, i = idx % inputs;
-    in[i * R + r] = r0 + r < n ? X[(r0 + r) * inputs + i] : 0.0f;
+  if constexpr (R < 64) {
+    for (uint32_t idx = threadIdx.x; idx < inputs * R; idx += blockDim.x) {
+      const uint32_t r = idx / inputs, i = idx % inputs;
+      in[i * R + r] = r0 + r < n ? X[(r0 + r) * inputs + i] : 0.0f;
+    }
+  } else {
+    struct __attribute__((packed, aligned(4))) Four {
+      float v[4];
+    };
+    for (uint32_t idx = threadIdx.x; idx < (inputs + 3) / 4 * R; idx += blockDim.x) {
+      const uint32_t r = idx % R, i = 4 * (idx / R);
+      const float *x = X + (r0 + r) * inputs + i;
+      Four f = {{0.0f, 0.0f, 0.0f, 0.0f}};
+      if (r0 + r < n) {
+        if (i + 4 <= inputs) {
+          f = *reinterpret_cast<const Four *>(x);
+        } else {
+          for (uint32_t k = 0; i + k < inputs; ++k) f.v[k] = x[k];
+        }
+      }
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k)
+        if (i + k < inputs) in[(i + k) * R + r] = f.v[k];
+    }
   }
 }
 
@@ -143,13 +169,13 @@ __global__ void __launch_bounds__(256) mlp_forward(const Shape s, const float *_
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const uint32_t width = s.inputs > s.hidden ? s.inputs : s.hidden;
   float *in = lds, *out = lds + width * R;
-  const float *weights = lds + 2 * width * R;
-  if (RESIDENT) read_weights(s, params, lds + 2 * width * R);
+  float *weights = out + s.hidden * R;
+  if (RESIDENT) read_weights(s, params, weights);
   const uint64_t r0 = (uint64_t)blockIdx.x * R;
   read_rows<R>(X, n, s.inputs, r0, in);
   __syncthreads();
   for (uint32_t l = 0; l <= s.layers; ++l) {
-    dense<R>(layer_of<RESIDENT>(s, l, params, weights), s.fan_in(l), s.fan_out(l), l < s.layers, in, out);
+    dense<R, false>(layer_of<RESIDENT>(s, l, params, weights), s.fan_in(l), s.fan_out(l), l < s.layers, in, out);
     __syncthreads();
     float *t = in;
     in = out;
@@ -198,8 +224,8 @@ __global__ void __launch_bounds__(gradient_threads(RESIDENT)) mlp_gradient(const
     read_rows<R>(X, n, s.inputs, r0, act);
     __syncthreads();
     for (uint32_t l = 0; l <= s.layers; ++l) {
-      dense<R>(layer_of<RESIDENT>(s, l, params, weights), s.fan_in(l), s.fan_out(l), l < s.layers, input_of(l),
-               l < s.layers ? input_of(l + 1) : GX, rows);
+      dense<R, true>(layer_of<RESIDENT>(s, l, params, weights), s.fan_in(l), s.fan_out(l), l < s.layers, input_of(l),
+                     l < s.layers ? input_of(l + 1) : GX, rows);
       __syncthreads();
     }
     // the output's error 2 (y - t) / n, and the squares
@@ -370,7 +396,7 @@ uint32_t gradient_lds(const Shape &s, uint32_t R, bool resident) {
               (resident ? s.lds_floats() : s.hidden * (kColumns + 1)));
 }
 uint32_t forward_lds(const Shape &s, uint32_t R, bool resident) {
-  return 4 * (2 * std::max(s.inputs, s.hidden) * R + (resident ? s.lds_floats() : 0));
+  return 4 * ((std::max(s.inputs, s.hidden) + s.hidden) * R + (resident ? s.lds_floats() : 0));
 }
 
 // The weights are kept in LDS where 16 rows' activations fit beside them (up to
@@ -399,14 +425,22 @@ dd_status reserve_parts(dd_mlp *net, uint32_t n) {
   return reserve(net->part, net->part_groups, gradient_groups(net->shape, n), net->count + 1);
 }
 
+// Rows per workgroup of the forward pass.  Its weights are kept in LDS where the
+// gradient's are and they fit; else a workgroup takes four rows.  Sixteen rows of up to
+// 16 units are too little work for a workgroup: many rows go 64 at a time (200000 rows
+// of 1 x 1 x 1 21.9 -> 8.6 us, of 5 x 8 x 1 26.6 -> 11.5, of 256 x 8 x 1 321 -> 210; one
+// launch per layer 10.4, 16.0 and 206).
+bool forward_resident(const Shape &s) { return resident(s) && forward_lds(s, 16, true) <= kResidentLds; }
+uint32_t forward_rows(const Shape &s, uint32_t n) {
+  if (!forward_resident(s)) return 4;
+  return s.hidden <= 16 && n >= 64 * 1024 && forward_lds(s, 64, true) <= kHalfLds ? 64 : 16;
+}
+
 dd_status forward(dd_mlp *net, const float *d_x, uint32_t n, float *d_y, hipStream_t s) {
   const Shape &sh = net->shape;
-  if (resident(sh))
-    hipLaunchKernelGGL((mlp_forward<16, true>), dim3(blocks_for(n, 16)), dim3(256), forward_lds(sh, 16, true), s, sh, d_x,
-                       n, net->params, d_y);
-  else
-    hipLaunchKernelGGL((mlp_forward<4, false>), dim3(blocks_for(n, 4)), dim3(256), forward_lds(sh, 4, false), s, sh, d_x,
-                       n, net->params, d_y);
+  const uint32_t R = forward_rows(sh, n);
+  auto kernel = R == 64 ? mlp_forward<64, true> : R == 16 ? mlp_forward<16, true> : mlp_forward<4, false>;
+  hipLaunchKernelGGL(kernel, dim3(blocks_for(n, R)), dim3(256), forward_lds(sh, R, R != 4), s, sh, d_x, n, net->params, d_y);
   MLP_HIP(hipGetLastError());
   return DD_OK;
 }

@@ -128,3 +128,27 @@ def test_largest_network_takes_bounded_memory(torch_cuda):
         assert free - torch.cuda.mem_get_info()[0] <= (512 << 20) + (4 << 20)  # and the allocator's granularity
     finally:
         lib.dd_mlp_destroy(h)
+
+
+# narrow networks over many rows, whose blocks have 64 rows from 65536 rows on, on both
+# sides of that line and of whole blocks; a wide input whose weights fit in LDS beside
+# the gradient's rows but not beside the forward pass's
+@pytest.mark.parametrize("shape,n", [((1, 1, 1), 65535), ((1, 1, 1), 65536), ((5, 8, 1), 65599), ((63, 16, 8), 65601),
+                                     ((12, 17, 2), 65540), ((256, 8, 1), 65602), ((254, 3, 2), 66001), ((256, 16, 1), 65537),
+                                     ((256, 39, 1), 50)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_forward_blocks(torch_cuda, shape, n):
+    torch = torch_cuda
+    lib, h, p, rng = network(shape, n)
+    try:
+        x = rng.standard_normal((n, shape[0])).astype(np.float32)
+        set_params(lib, h, p)
+        dx = torch.from_numpy(x).cuda()
+        dy = torch.full((n + 64,), 7.0, dtype=torch.float32, device="cuda")
+        check(lib.dd_mlp_forward(h, dx.data_ptr(), n, dy.data_ptr(), None))
+        want, _ = mlp.forward(p.astype(np.float64), x.astype(np.float64), *shape)
+        got = dy.cpu().numpy()
+        assert np.max(np.abs(got[:n] - want)) <= 1e-5 * max(1.0, np.max(np.abs(want)))
+        assert np.all(got[n:] == 7.0)
+    finally:
+        lib.dd_mlp_destroy(h)
