@@ -104,6 +104,15 @@ def _f32_ptr(a: np.ndarray):
     return a.ctypes.data_as(ctypes.POINTER(ctypes.c_float))
 
 
+# The kernel forms of dd_form, in its order.
+FORMS = ("direct", "groups", "staged", "patterns", "matrix", "pairs", "whole")
+
+
+def _launch_dict(i) -> dict:
+    return {"form": FORMS[i.form], "rows_per_barrier": i.rows_per_barrier, "lds_bytes": i.lds_bytes,
+            "many_windows": bool(i.many_windows), "tiles_per_run": i.tiles_per_run}
+
+
 class Plan:
     """A dd_plan: observation, padding, device-resident tables, launches."""
 
@@ -175,6 +184,15 @@ class Plan:
         c = _lib.DDConf()
         check(self.lib.dd_plan_get_conf(self.handle, mode, ctypes.byref(c)))
         return Conf.from_c(c)
+
+    def launch_info(self, mode: int, conf: Optional[Conf] = None) -> dict:
+        """How the launches of `mode` run under `conf` (None: the plan's
+        configuration): the kernel's form (one of FORMS), the rows staged per
+        barrier and the LDS."""
+        i = _lib.DDLaunchInfo()
+        c = None if conf is None else ctypes.byref(conf.to_c())
+        check(self.lib.dd_plan_get_launch_info(self.handle, mode, c, ctypes.byref(i)))
+        return _launch_dict(i)
 
     def set_zapped_channels(self, zapped: Sequence[int]) -> None:
         flags = np.zeros(self.pad(self.obs.nr_channels, 4), dtype=np.uint32)
@@ -327,6 +345,12 @@ class Batch:
 
     def run_per_job(self, stream: int = 0) -> None:
         check(self.lib.dd_batch_run_per_job(self.handle, stream or None))
+
+    def launch_info(self, mode: int) -> dict:
+        """The kernel that runs the batch's jobs of `mode`, as Plan.launch_info."""
+        i = _lib.DDLaunchInfo()
+        check(self.lib.dd_batch_get_launch_info(self.handle, mode, ctypes.byref(i)))
+        return _launch_dict(i)
 
     def job_placement(self, job: int) -> dict:
         """Where job `job` runs: {"beside": beside the batch kernels, with the

@@ -125,6 +125,16 @@ class DDBatchInfo(ctypes.Structure):
     ]
 
 
+class DDLaunchInfo(ctypes.Structure):
+    _fields_ = [
+        ("form", c_uint32),
+        ("rows_per_barrier", c_uint32),
+        ("lds_bytes", c_uint32),
+        ("many_windows", c_uint32),
+        ("tiles_per_run", c_uint32),
+    ]
+
+
 class DDStreamInfo(ctypes.Structure):
     _fields_ = [
         ("slots", c_uint32),
@@ -164,6 +174,7 @@ PROTOTYPES = {
     "dd_plan_set_input_bits": (c_int, [c_void_p, c_uint32]),
     "dd_plan_set_conf": (c_int, [c_void_p, c_int, POINTER(DDConf)]),
     "dd_plan_get_conf": (c_int, [c_void_p, c_int, POINTER(DDConf)]),
+    "dd_plan_get_launch_info": (c_int, [c_void_p, c_int, POINTER(DDConf), POINTER(DDLaunchInfo)]),
     "dd_plan_set_zapped_channels": (c_int, [c_void_p, POINTER(c_uint32)]),
     "dd_plan_set_beam_mapping": (c_int, [c_void_p, POINTER(c_uint32), POINTER(c_uint32)]),
     "dd_plan_set_shifts": (c_int, [c_void_p, POINTER(c_float), POINTER(c_float)]),
@@ -196,6 +207,7 @@ PROTOTYPES = {
     "dd_batch_run_mode": (c_int, [c_void_p, c_int, c_void_p]),
     "dd_batch_run_per_job": (c_int, [c_void_p, c_void_p]),
     "dd_batch_get_info": (c_int, [c_void_p, POINTER(DDBatchInfo)]),
+    "dd_batch_get_launch_info": (c_int, [c_void_p, c_int, POINTER(DDLaunchInfo)]),
     "dd_batch_run_static": (c_int, [c_void_p, c_void_p]),
     "dd_batch_set_paired_step_two": (c_int, [c_void_p, c_int]),
     "dd_batch_get_job_placement": (c_int, [c_void_p, c_uint32, POINTER(c_uint32), POINTER(c_uint32)]),

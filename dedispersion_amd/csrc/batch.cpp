@@ -737,6 +737,21 @@ dd_status dd_batch_set_paired_step_two(dd_batch *batch, int enable) {
   return DD_OK;
 }
 
+dd_status dd_batch_get_launch_info(dd_batch *batch, dd_mode mode, dd_launch_info *info) {
+  if (!batch || !info || (int)mode < 0 || (int)mode > 2) return fail(DD_ERR_INVALID_ARGUMENT, "invalid argument");
+  dd_status s = build(batch);
+  if (s != DD_OK) return s;
+  const KindQueue &k = batch->q[mode];
+  if (k.n_tiles == 0) return fail(DD_ERR_NOT_READY, "no job of this mode in the batch kernels");
+  *info = info_of(k.g);
+  for (const U8Launch &L : k.u8) info->rows_per_barrier = std::max(info->rows_per_barrier, L.g.unroll);
+  for (const F32Launch &L : k.f32) {
+    info->rows_per_barrier = std::max(info->rows_per_barrier, L.g.unroll);
+    if (k.g.whole) info->tiles_per_run = L.k.tiles_per_run;
+  }
+  return DD_OK;
+}
+
 dd_status dd_batch_get_job_placement(dd_batch *batch, uint32_t job, uint32_t *beside, uint32_t *compact) {
   if (!batch || !beside || !compact) return fail(DD_ERR_INVALID_ARGUMENT, "null argument");
   if (job >= batch->jobs.size()) return fail(DD_ERR_INVALID_ARGUMENT, "job index out of range");

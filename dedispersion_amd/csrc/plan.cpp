@@ -877,6 +877,22 @@ dd_status prepare_step_one_f32(dd_plan *plan, const dd_conf &c, const float *d_i
   return DD_OK;
 }
 
+dd_launch_info info_of(const Geometry &g) {
+  dd_launch_info info{};
+  info.form = g.pairs          ? DD_FORM_PAIRS
+              : g.whole        ? DD_FORM_WHOLE
+              : g.staged == 2  ? DD_FORM_PATTERNS
+              : g.matrix       ? DD_FORM_MATRIX
+              : g.staged       ? DD_FORM_STAGED
+              : g.local        ? DD_FORM_GROUPS
+                               : DD_FORM_DIRECT;
+  info.rows_per_barrier = g.unroll;
+  info.lds_bytes = g.lds_bytes;
+  info.many_windows = g.wide;
+  info.tiles_per_run = 1;
+  return info;
+}
+
 dd_status run(const U8Launch &L, hipStream_t stream) {
   if (L.g.staged == 2) {
     DD_HIP(launch_rowsum_u8_factored(L.k, L.g, stream));
@@ -1093,6 +1109,15 @@ dd_status dd_plan_get_conf(const dd_plan *plan, dd_mode mode, dd_conf *conf) {
   if (!plan || !conf || (int)mode < 0 || (int)mode > 2) return fail(DD_ERR_INVALID_ARGUMENT, "invalid argument");
   *conf = plan->conf[mode];
   return DD_OK;
+}
+
+dd_status dd_plan_get_launch_info(dd_plan *plan, dd_mode mode, const dd_conf *conf, dd_launch_info *info) {
+  if (!plan || !info || (int)mode < 0 || (int)mode > 2) return fail(DD_ERR_INVALID_ARGUMENT, "invalid argument");
+  if (mode != DD_SINGLE_STEP && !plan->two_step) return fail(DD_ERR_INVALID_ARGUMENT, "plan has no subband path");
+  Geometry g;
+  const dd_status s = geometry_of(plan, mode, conf ? *conf : plan->conf[mode], g);
+  if (s == DD_OK) *info = info_of(g);
+  return s;
 }
 
 dd_status dd_plan_set_zapped_channels(dd_plan *plan, const uint32_t *zapped) {

@@ -164,6 +164,9 @@ enum class ByteKernel { kByRule, kVector, kMatrix };
 // matrix form has no such shape) and the LDS that it needs.
 void set_byte_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, ByteKernel kernel, Geometry &g);
 
+// What dd_plan_get_launch_info and dd_batch_get_launch_info say of a geometry.
+dd_launch_info info_of(const Geometry &g);
+
 // One prepared launch of a mode: kernel parameters, geometry and grid.
 struct U8Launch {
   RowSumU8Params k{};

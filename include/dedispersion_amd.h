@@ -209,6 +209,30 @@ dd_status dd_plan_set_step_one_shifts(dd_plan *plan, dd_step_one_shifts delays);
 dd_status dd_plan_set_conf(dd_plan *plan, dd_mode mode, const dd_conf *conf);
 dd_status dd_plan_get_conf(const dd_plan *plan, dd_mode mode, dd_conf *conf);
 
+/* How the launches of a mode run: the kernel's form, chosen from the
+ * configuration, the sizes, the delays and the input's type.  Every form gives
+ * the same sums. */
+typedef enum dd_form {
+  DD_FORM_DIRECT = 0,   /* rows read through the caches */
+  DD_FORM_GROUPS = 1,   /* rows staged in LDS, one group at a time */
+  DD_FORM_STAGED = 2,   /* rows staged in LDS by the double-buffered pipeline */
+  DD_FORM_PATTERNS = 3, /* channel-block patterns (local 3) */
+  DD_FORM_MATRIX = 4,   /* staged byte rows summed on the matrix cores */
+  DD_FORM_PAIRS = 5,    /* a batch's step two: uint16 sums added in pairs first */
+  DD_FORM_WHOLE = 6     /* a batch's step two: all uint16 rows of a tile in LDS at once */
+} dd_form;
+typedef struct dd_launch_info {
+  uint32_t form;             /* dd_form */
+  uint32_t rows_per_barrier; /* rows staged per barrier: the configuration's unroll, or fewer */
+  uint32_t lds_bytes;        /* dynamic LDS per workgroup */
+  uint32_t many_windows;     /* matrix form: rows may take more than one window of 32 samples */
+  uint32_t tiles_per_run;    /* whole rows: sample tiles that a workgroup sums one after another, else 1 */
+} dd_launch_info;
+/* The launch of `mode` under `conf` (NULL: the plan's configuration), for input at
+ * a multiple of 4 bytes (bytes elsewhere never take the matrix form).  Fails as
+ * dd_plan_set_conf does where the configuration cannot run. */
+dd_status dd_plan_get_launch_info(dd_plan *plan, dd_mode mode, const dd_conf *conf, dd_launch_info *info);
+
 /* Zapped channels, the reference's uint32 flags [pad(C, padding/4)]
  * (src/DedispersionTest.cpp:120); non-zero = zapped.  Host pointer.
  * Compacted into device-resident lists of the live channels (per subband for
@@ -410,6 +434,9 @@ dd_status dd_batch_run_mode(dd_batch *batch, dd_mode mode, void *stream);
  * configuration and the float intermediate of the reference layout. */
 dd_status dd_batch_run_per_job(dd_batch *batch, void *stream);
 dd_status dd_batch_get_info(dd_batch *batch, dd_batch_info *info);
+/* The one kernel that runs all jobs of `mode` in the batch kernels (the largest
+ * of its jobs' rows_per_barrier); DD_ERR_NOT_READY when there are none. */
+dd_status dd_batch_get_launch_info(dd_batch *batch, dd_mode mode, dd_launch_info *info);
 /* Where job `job` (in the order of the dd_batch_add_* calls) runs: beside = 1
  * when it runs beside the batch kernels as its plan's own launches (its
  * intermediate then holds the reference's floats); compact = 1 when its

@@ -1,0 +1,232 @@
+"""Which form of a kernel runs, and that each gives the oracle's sums bit for bit
+(integer sums: no tolerance).  Every case names the form it is meant for and fails
+where another runs: the matrix form of the byte row sums at the edges of its sets of
+four rows, of its blocks of samples and of its windows, over packed rows, and its
+fallback for input that is not at a dword; batches whose jobs agree on a form,
+disagree, or cannot take it, in the persistent and in the chunked launches."""
+import numpy as np
+import pytest
+
+import oracle
+from dedispersion_amd import DD_SINGLE_STEP, DD_STEP_ONE, DD_STEP_TWO, Batch, Conf, DDError, Plan, workloads
+from tests.conftest import host_threads
+from tests.gpu_helpers import compare_rows, stream_of, zapped_flags
+from tests.packing import pack_rows, random_values
+
+pytestmark = pytest.mark.gpu
+
+BIG, MID, SMALL, TINY = (Conf(64, 8, 16, 8, 16, 1), Conf(64, 4, 8, 8, 8, 1), Conf(64, 4, 16, 4, 8, 1),
+                         Conf(64, 8, 4, 4, 16, 1))
+
+
+def beam(channels, samples, dms, step, zapped=(), bits=8, padding=128, offset=0, beams=1, seed=7, subbands=1, coarse=0,
+         coarse_step=0.0):
+    """One job: its plan, its input `offset` bytes past a dword, its buffers and the oracle's results."""
+    import torch
+
+    w = workloads.tiny(channels=channels, samples=samples, dms=dms, step=step, beams=beams, sbeams=beams, min_freq=1250.0,
+                       bandwidth=300.0 / channels, zapped=zapped, seed=seed, subbands=subbands, coarse=coarse,
+                       coarse_step=coarse_step)
+    plan = Plan(w.obs, padding, input_bits=bits)
+    flags = zapped_flags(plan, zapped)
+    plan.set_zapped_channels(flags)
+    orc = oracle.Oracle(w.obs, padding, threads=host_threads(), input_bits=bits)
+    z = plan.sizes
+    pitch, length = (z.sub_in_pitch, z.nr_dispersed_samples_subbanding) if coarse else (z.in_pitch, z.nr_dispersed_samples)
+    host = pack_rows(random_values(np.random.default_rng(seed + samples), beams * channels, length, bits), bits, pitch).ravel()
+    room = torch.zeros(host.size + offset, dtype=torch.uint8, device="cuda")
+    room[offset:].copy_(torch.from_numpy(host))
+    mid = torch.full((max(z.intermediate_elements, 1),), -1.0, dtype=torch.float32, device="cuda")
+    out = torch.full((z.sub_output_elements if coarse else z.output_elements,), -1.0, dtype=torch.float32, device="cuda")
+    want = orc.step_two(orc.step_one(host, flags).ravel()) if coarse else orc.dedispersion(host, flags)
+    return {"plan": plan, "input": room[offset:], "room": room, "mid": mid, "out": out, "want": want, "samples": samples,
+            "two_step": bool(coarse)}
+
+
+def verify(job, what):
+    got = job["out"].cpu().numpy().reshape(job["want"].shape)
+    compare_rows(got, job["want"], job["samples"], what)
+    assert np.all(got[..., job["samples"]:] == -1.0)
+
+
+# channels, zapped, samples, dms, step, bits, padding, conf, several windows per row
+MATRIX = [
+    *[(72, tuple(range(1, 1 + k)), 1024, 64, 0.12, 8, 128, BIG, False) for k in range(5)],  # 72 - k rows
+    *[(70, (), s, 37, 0.12, 8, 0, BIG, False) for s in (1, 127, 129, 1023, 1025, 2100)],
+    *[(66, (3,), 700, 33, 0.1, 8, 128, c, False) for c in (MID, SMALL, TINY)],
+    # spreads over a wavefront's eight DMs of the lowest channel: one window takes 17 and 7 + 8
+    *[(300, (), 900, 40, step, 8, 128, BIG, step > 0.22) for step in (0.19, 0.215, 0.23, 0.32, 0.4)],
+    (300, (9,), 900, 37, 0.4, 8, 0, MID, True),
+    *[(130, (7, 8), 1500, 40, 0.12, bits, pad, c, False) for bits in (1, 2, 4) for pad in (0, 128) for c in (BIG, SMALL)],
+    *[(300, (7,), 1500, 40, 0.35, bits, 0, BIG, True) for bits in (1, 2, 4)],
+]
+
+
+@pytest.mark.parametrize("case", MATRIX, ids=lambda c: "-".join(str(v) for v in (c[0] - len(c[1]), *c[2:7], c[7].threads_d1,
+                                                                               c[7].items_d0, c[7].items_d1)))
+def test_matrix(torch_cuda, case):
+    channels, zapped, samples, dms, step, bits, padding, conf, wide = case
+    job = beam(channels, samples, dms, step, zapped, bits, padding, beams=2)
+    job["plan"].set_conf(DD_SINGLE_STEP, conf)
+    info = job["plan"].launch_info(DD_SINGLE_STEP)
+    assert info["form"] == "matrix" and info["many_windows"] == wide, info
+    job["plan"].dedisperse(job["input"].data_ptr(), job["out"].data_ptr(), stream=stream_of(torch_cuda))
+    verify(job, f"{case}")
+
+
+@pytest.mark.parametrize("offset", [0, 1, 2, 3])
+@pytest.mark.parametrize("two_step", [False, True])
+def test_input_off_a_dword(torch_cuda, two_step, offset):
+    """The same call at and past a dword: the matrix form, and the vector form."""
+    job = beam(160, 640, 24, 0.12, offset=offset, **(dict(subbands=2, coarse=16, coarse_step=0.1) if two_step else {}))
+    mode = DD_STEP_ONE if two_step else DD_SINGLE_STEP
+    batch = Batch()
+    add(batch, job)
+    batch.set_conf(mode, MID)
+    assert batch.launch_info(mode)["form"] == ("staged" if offset else "matrix")
+    batch.run(stream=stream_of(torch_cuda))
+    verify(job, f"batch, {offset}")
+    job["out"].fill_(-1.0)
+    plan = job["plan"]
+    plan.set_conf(mode, MID)
+    assert plan.launch_info(mode)["form"] == "matrix"  # of input at a dword
+    if two_step:
+        plan.step_one(job["input"].data_ptr(), job["mid"].data_ptr(), stream=stream_of(torch_cuda))
+        plan.step_two(job["mid"].data_ptr(), job["out"].data_ptr(), stream=stream_of(torch_cuda))
+    else:
+        plan.dedisperse(job["input"].data_ptr(), job["out"].data_ptr(), stream=stream_of(torch_cuda))
+    verify(job, f"plan, {offset}")
+
+
+def add(batch, job):
+    if job["two_step"]:
+        batch.add_two_step(job["plan"], job["input"].data_ptr(), job["mid"].data_ptr(), job["out"].data_ptr(), keep=(job,))
+    else:
+        batch.add_single_step(job["plan"], job["input"].data_ptr(), job["out"].data_ptr(), keep=(job,))
+
+
+NARROW = dict(channels=300, samples=2100, dms=70, step=0.1)  # one window per row
+SEVERAL = dict(channels=300, samples=900, dms=40, step=0.35)  # ... more for some
+SPREAD = dict(channels=300, samples=900, dms=40, step=1.3)  # the vector form's
+FEW = dict(channels=40, samples=900, dms=40, step=0.1)  # too few rows for the matrix form
+
+
+def two(j, subbands=3, coarse=24):
+    """A job in two steps whose coarse DMs have the steps, and whose subbands the rows, of a single-step job."""
+    return dict(j, channels=j["channels"] * subbands, dms=7, step=0.3, subbands=subbands, coarse=coarse,
+                coarse_step=j["step"] * (subbands if j["step"] > 1.0 else 1))
+
+
+SINGLE_BATCHES = [
+    ("one", [NARROW], "matrix", False),
+    ("agree", [NARROW, dict(NARROW, zapped=(5,), samples=333), dict(NARROW, beams=2, dms=9)], "matrix", False),
+    ("several windows", [NARROW, SEVERAL], "matrix", True),
+    ("packed with bytes", [NARROW, dict(NARROW, bits=2, padding=0), dict(SEVERAL, bits=1), dict(NARROW, bits=4)], "matrix", True),
+    ("mostly matrix", [dict(NARROW, samples=9000), SPREAD], "matrix", True),
+    ("mostly vector", [NARROW, dict(SPREAD, samples=30000)], "staged", False),
+    ("few rows", [FEW, FEW], "staged", False),
+    ("one off a dword", [dict(NARROW, samples=9000), dict(NARROW, offset=1)], "staged", False),
+    ("packed, one off a dword", [dict(NARROW, bits=2), dict(NARROW, bits=2, offset=3, samples=70)], "staged", False),
+]
+
+
+@pytest.mark.parametrize("case", SINGLE_BATCHES, ids=lambda c: c[0])
+def test_single_step_batch(torch_cuda, case):
+    name, shapes, form, wide = case
+    jobs = [beam(**s, seed=20 + k) for k, s in enumerate(shapes)]
+    batch = Batch()
+    for j in jobs:
+        add(batch, j)
+    info = batch.launch_info(DD_SINGLE_STEP)
+    assert info["form"] == form and info["many_windows"] == wide, info
+    for graph in (False, True):
+        for j in jobs:
+            j["out"].fill_(-1.0)
+        batch.run(use_graph=graph, stream=stream_of(torch_cuda))
+        for k, j in enumerate(jobs):
+            verify(j, f"{name}, graph {graph}, job {k}")
+
+
+@pytest.mark.parametrize("chunks", [0, 2])
+@pytest.mark.parametrize("compact", [True, False])
+@pytest.mark.parametrize("case", [c for c in SINGLE_BATCHES if c[0] not in ("few rows", "mostly vector")], ids=lambda c: c[0])
+def test_two_step_batch(torch_cuda, case, compact, chunks):
+    """Step one in the persistent launch and in the chunks' lists, as floats and as uint16 sums."""
+    name, shapes, form, wide = case
+    shapes = [dict(two(s), samples=min(s["samples"], 3000), zapped=s.get("zapped", (1,)), seed=40 + k)
+              for k, s in enumerate(shapes)]
+    if compact:  # 257 live channels per subband are the most whose sums fit 16 bits
+        shapes = [dict(s, channels=3 * 250) for s in shapes]
+    jobs = [beam(**s) for s in shapes]
+    batch = Batch()
+    for j in jobs:
+        add(batch, j)
+    batch.set_compact_intermediate(compact)
+    batch.set_pipeline(chunks)
+    assert batch.info()["compact_intermediate"] == int(compact)
+    info = batch.launch_info(DD_STEP_ONE)
+    assert info["form"] == form, info
+    for graph in (False, True):
+        for j in jobs:
+            j["out"].fill_(-1.0)
+        batch.run(use_graph=graph, stream=stream_of(torch_cuda))
+        for k, j in enumerate(jobs):
+            verify(j, f"{name}, chunks {chunks}, graph {graph}, job {k}")
+
+
+def test_queries_refuse_what_cannot_run(torch_cuda):
+    job = beam(64, 100, 8, 0.5)
+    with pytest.raises(DDError):
+        job["plan"].launch_info(DD_SINGLE_STEP, Conf(32, 4, 4, 4, 4, 1))
+    with pytest.raises(DDError):
+        job["plan"].launch_info(DD_STEP_TWO)
+    batch = Batch()
+    add(batch, job)
+    batch.launch_info(DD_SINGLE_STEP)
+    with pytest.raises(DDError):
+        batch.launch_info(DD_STEP_TWO)
+
+
+# subbands, channels per subband, samples, fine DMs, coarse DMs, step, shape, form, tiles per run
+STEP_TWO = [
+    (31, 3, 700, 19, 3, 0.2, Conf(64, 8, 8, 4, 2, 1), "whole", 1),
+    (33, 3, 700, 19, 3, 0.7, Conf(64, 8, 4, 4, 2, 1), "whole", 1),
+    (33, 3, 700, 19, 3, 0.7, Conf(64, 8, 8, 4, 2, 1), "staged", 1),  # rows that two workgroups' LDS has no room for
+    (66, 3, 700, 19, 3, 0.2, Conf(64, 8, 4, 2, 2, 1), "whole", 1),
+    (5, 257, 700, 19, 3, 0.3, Conf(64, 8, 8, 4, 2, 1), "whole", 1),
+    (7, 2, 1100, 9, 2, 0.7, Conf(64, 2, 16, 1, 2, 1), "whole", 1),
+    (60, 2, 1100, 64, 2, 0.2, Conf(64, 8, 16, 8, 2, 1), "staged", 1),
+    (2, 2, 8200, 32, 600, 0.5, Conf(64, 8, 8, 4, 2, 1), "whole", 2),   # the last run cut short
+]
+
+
+@pytest.mark.parametrize("chunks", [0, 2])
+@pytest.mark.parametrize("case", STEP_TWO, ids=lambda c: "-".join(str(v) for v in (*c[:6], c[6].items_d0)))
+def test_whole_rows(torch_cuda, case, chunks):
+    subbands, per, samples, fine, coarse, step, conf, form, run = case
+    job = beam(subbands * per, samples, fine, step, (1,), subbands=subbands, coarse=coarse, coarse_step=0.05)
+    batch = Batch()
+    add(batch, job)
+    batch.set_conf(DD_STEP_TWO, conf)
+    batch.set_pipeline(chunks)
+    info = batch.launch_info(DD_STEP_TWO)
+    assert info["form"] == form and info["tiles_per_run"] == run, info
+    batch.run(stream=stream_of(torch_cuda))
+    verify(job, f"{case}")
+
+
+@pytest.mark.parametrize("chunks", [0, 2])
+@pytest.mark.parametrize("several", ["all have room", "one has none"])
+def test_whole_rows_of_several_jobs(torch_cuda, several, chunks):
+    """One step-two kernel for the batch: whole rows only where every job's fit."""
+    shapes = [(16, 700, 32, 3), (5, 2100, 9, 4), (16 if several == "all have room" else 90, 1030, 33, 2)]
+    jobs = [beam(s * 4, samples, fine, 0.3, (2,), subbands=s, coarse=coarse, coarse_step=2.0, seed=60 + k)
+            for k, (s, samples, fine, coarse) in enumerate(shapes)]
+    batch = Batch()
+    for j in jobs:
+        add(batch, j)
+    batch.set_pipeline(chunks)
+    assert batch.launch_info(DD_STEP_TWO)["form"] == ("whole" if several == "all have room" else "staged")
+    batch.run(stream=stream_of(torch_cuda))
+    for k, j in enumerate(jobs):
+        verify(j, f"{several}, chunks {chunks}, job {k}")
