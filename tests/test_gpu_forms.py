@@ -192,7 +192,7 @@ STEP_TWO = [
     (31, 3, 700, 19, 3, 0.2, Conf(64, 8, 8, 4, 2, 1), "whole", 1),
     (33, 3, 700, 19, 3, 0.7, Conf(64, 8, 4, 4, 2, 1), "whole", 1),
     (33, 3, 700, 19, 3, 0.7, Conf(64, 8, 8, 4, 2, 1), "staged", 1),  # rows that two workgroups' LDS has no room for
-    (66, 3, 700, 19, 3, 0.2, Conf(64, 8, 4, 2, 2, 1), "whole", 1),
+    (60, 3, 700, 19, 3, 0.2, Conf(64, 8, 4, 2, 2, 1), "whole", 1),
     (5, 257, 700, 19, 3, 0.3, Conf(64, 8, 8, 4, 2, 1), "whole", 1),
     (7, 2, 1100, 9, 2, 0.7, Conf(64, 2, 16, 1, 2, 1), "whole", 1),
     (60, 2, 1100, 64, 2, 0.2, Conf(64, 8, 16, 8, 2, 1), "staged", 1),
