@@ -31,17 +31,33 @@ dd_status hip_fail(hipError_t e, const char *what) {
 
 namespace {
 
-// Whether the matrix-core byte kernel sums `rows` rows faster than the vector
-// one, with `dms` DMs per wavefront, by the windows per row on average:
-// its products grow with the windows, the vector kernel's additions do not;
-// eight DMs share the operands that four read; above 257 rows the vector kernel
-// spills its 16-bit sums to 32 bits.  Measured (us, matrix against vector form,
-// each at its best shape): 1024 DMs x 24576 samples, 1.0 windows: 48 rows 45
-// and 45, 64 rows 53 and 56, 256 rows 144 and 175, 512 rows 264 and 399; 512
-// DMs, 256 rows: 1.4 windows 102 and 101, 2.0 windows 119 and 115; 1536 rows: 1.1
-// windows 444 and 632, 1.4 windows 543 and 633, 2.0 windows 657 and 635.
-bool matrix_is_faster(uint32_t rows, uint32_t dms, const ShiftTable &t) {
-  return rows >= 64 && t.mean_windows(dms) <= (dms < 8 ? 1.1f : rows > 257 ? 1.6f : 1.25f);
+// Whether the matrix-core byte kernel sums `rows` rows faster than the vector one
+// under configuration c with `unroll` rows per barrier.
+//
+// By the windows per row on average: its products grow with the windows, the
+// vector kernel's additions do not; eight DMs share the operands that four read;
+// above 257 rows the vector kernel spills its 16-bit sums to 32 bits.  Measured (us,
+// matrix against vector form, each at its best shape): 1024 DMs x 24576 samples, 1.0
+// windows: 48 rows 45 and 45, 64 rows 53 and 56, 256 rows 144 and 175, 512 rows 264
+// and 399; 512 DMs, 256 rows: 1.4 windows 102 and 101, 2.0 windows 119 and 115; 1536
+// rows: 1.1 windows 444 and 632, 1.4 windows 543 and 633, 2.0 windows 657 and 635.
+//
+// By the work between two barriers: rows go in sets of four, and what a set costs
+// beside its products is shared by the wavefront's sums.  Time of the matrix form in
+// that of the vector form, 512 DMs x 8192 samples, 1.0 windows, over 1536 and 96
+// rows: 1 or 2 rows per barrier 0.98-3.5 in all 42 shapes; by samples x DMs x rows per
+// barrier of a lane, where every wavefront stages two rows: 64 1.01-1.07, 128 0.88-0.99,
+// 256 0.72-0.99, 512 0.68-0.93, more 0.54-0.77; where not: 64 and 128 1.03-1.49, 256
+// 0.93-1.08, 512 0.75-0.95, 1024 0.66-0.75.  At 1.4 windows over 1536 rows, eight DMs:
+// two rows each 256 1.02, 512 0.84-1.03, more 0.73-0.97; else 512 0.99-1.13, 1024 0.87.
+bool matrix_is_faster(uint32_t rows, const dd_conf &c, uint32_t unroll, const ShiftTable &t) {
+  if (rows < 64 || unroll < 4) return false;
+  const bool full = unroll >= kStagedSlotsPerWave * c.threads_d1;
+  const uint32_t work = c.items_d0 * c.items_d1 * unroll * unroll / roundup(unroll, 4);
+  if (work < (full ? 128 : 512)) return false;
+  const bool much = work >= (full ? 512 : 1024);
+  const float most = c.items_d1 < 8 ? 1.1f : rows > 257 ? (much ? 1.6f : 1.2f) : much ? 1.25f : 1.1f;
+  return t.mean_windows(c.items_d1) <= most;
 }
 
 uint32_t cps(const dd_plan *p) { return p->obs.nr_channels / p->obs.nr_subbands; }
@@ -426,15 +442,18 @@ void set_byte_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, ByteKerne
       return 4 * (4 * slots + 3 * u * ((g.win + kU8MatrixReach) / 4) + 2 * (roundup(u, 4) + 4) * (tile + c.threads_d1)) + past;
     return 4 * (roundup(2 * slots, 4) + 2 * u * g.win + 2 * u * tile);
   };
+  auto fitting = [&](bool matrix) {
+    uint32_t u = std::min(c.unroll, kStagedSlotsPerWave * c.threads_d1);
+    while (u > 1 && lds_of(u, matrix) > p->max_lds) --u;
+    return u;
+  };
   const bool shaped = (c.items_d1 == 4 || c.items_d1 == 8) && g.win <= kU8MatrixWindow && lds_of(1, true) <= p->max_lds;
   g.matrix = shaped && (kernel == ByteKernel::kMatrix ||
-                        (kernel == ByteKernel::kByRule && matrix_is_faster(slots, c.items_d1, t)));
+                        (kernel == ByteKernel::kByRule && matrix_is_faster(slots, c, fitting(true), t)));
   // one window takes the first DM's shift modulo 8, the spread and the block's 8 samples
   g.wide = g.matrix && t.max_spread(c.items_d1) + 7 + 7 >= 32;
-  uint32_t unroll = std::min(c.unroll, kStagedSlotsPerWave * c.threads_d1);
-  while (unroll > 1 && lds_of(unroll, g.matrix) > p->max_lds) --unroll;
-  g.unroll = unroll;
-  g.lds_bytes = lds_of(unroll, g.matrix);
+  g.unroll = fitting(g.matrix);
+  g.lds_bytes = lds_of(g.unroll, g.matrix);
 }
 
 namespace {
@@ -457,7 +476,10 @@ dd_conf conf_of(uint32_t wavefronts, uint32_t items_d0, uint32_t items_d1, uint3
 // to the first (workgroups share a compute unit's time where two fit on it).
 // Measured at 0.2 pc/cc over 128-1536 rows, 64-2048 DMs and 2048-24576 samples:
 // the shape of least per_row x rounds is the fastest of all shapes, or within 4%
-// of it.
+// of it.  Bytes in the vector form take the matrix form's shapes: by its own times
+// at 0.2 pc/cc (0.45, 0.285, 0.19, 0.142, 0.125) it would take smaller ones, up to
+// 10% faster there but slower where windows are wide or rows few (979 rows, 243 DMs x
+// 11236 samples at 4.3 pc/cc 208 and 348 us; 7 rows, 606 DMs x 4851 6.9 and 9.3).
 struct Shape {
   uint32_t items_d0, items_d1;
   float per_row, again;
@@ -509,11 +531,11 @@ dd_conf default_conf(const dd_plan *p, dd_mode mode) {
   const uint32_t samples = single ? z.nr_samples : z.nr_samples_step_one;
   const uint64_t slices = single ? o.nr_synthesized_beams : (uint64_t)o.nr_beams * o.nr_subbands;
   if (single || rows >= 64) {
-    dd_conf c = floats ? best_shape(kFloatShapes, true, samples, dms, slices, cus)
-                       : best_shape(kByteShapes, false, samples, dms, slices, cus);
+    if (floats) return best_shape(kFloatShapes, true, samples, dms, slices, cus);
+    dd_conf c = best_shape(kByteShapes, false, samples, dms, slices, cus);
     // the vector form keeps four copies of a byte row
-    const ShiftTable &t = single ? p->ish_single : p->ish_one;
-    if (!floats && c.items_d1 >= 4 && !matrix_is_faster(rows, c.items_d1, t))
+    Geometry g;
+    if (c.items_d1 >= 4 && (geometry_of(p, mode, c, g) != DD_OK || !g.matrix))
       c.unroll = c.items_d0 == 16 ? 4 : c.items_d0 == 8 ? 8 : 16;
     return c;
   }

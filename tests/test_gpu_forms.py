@@ -56,7 +56,7 @@ MATRIX = [
     *[(66, (3,), 700, 33, 0.1, 8, 128, c, False) for c in (MID, SMALL, TINY)],
     # spreads over a wavefront's eight DMs of the lowest channel: one window takes 17 and 7 + 8
     *[(300, (), 900, 40, step, 8, 128, BIG, step > 0.22) for step in (0.19, 0.215, 0.23, 0.32, 0.4)],
-    (300, (9,), 900, 37, 0.4, 8, 0, MID, True),
+    (300, (9,), 900, 37, 0.4, 8, 0, Conf(64, 4, 16, 8, 8, 1), True),
     *[(130, (7, 8), 1500, 40, 0.12, bits, pad, c, False) for bits in (1, 2, 4) for pad in (0, 128) for c in (BIG, SMALL)],
     *[(300, (7,), 1500, 40, 0.35, bits, 0, BIG, True) for bits in (1, 2, 4)],
 ]
@@ -230,3 +230,37 @@ def test_whole_rows_of_several_jobs(torch_cuda, several, chunks):
     batch.run(stream=stream_of(torch_cuda))
     for k, j in enumerate(jobs):
         verify(j, f"{several}, chunks {chunks}, job {k}")
+
+
+# channels, dms, shape, the form, its rows per barrier: sets of four rows per barrier and
+# enough work between two barriers for the matrix form, else the vector form, whose
+# row list takes half the LDS
+ROWS_PER_BARRIER = [
+    *[(160, 64, Conf(64, t1, i0, i1, u, 1), "staged", u) for t1, i0, i1 in ((8, 16, 8), (4, 8, 4), (1, 4, 8)) for u in (1, 2)],
+    (160, 64, Conf(64, 8, 16, 8, 3, 1), "staged", 3),
+    (160, 64, Conf(64, 8, 16, 8, 4, 1), "matrix", 4),
+    (160, 64, Conf(64, 8, 8, 8, 4, 1), "staged", 4),
+    (160, 64, Conf(64, 8, 8, 8, 8, 1), "matrix", 8),
+    (160, 64, Conf(64, 8, 4, 4, 8, 1), "staged", 8),
+    (160, 64, Conf(64, 8, 4, 4, 16, 1), "matrix", 16),
+    (160, 64, Conf(64, 4, 4, 4, 8, 1), "matrix", 8),
+    (160, 64, Conf(64, 2, 8, 4, 4, 1), "matrix", 4),
+    (160, 64, Conf(64, 2, 4, 4, 4, 1), "staged", 4),
+    (9000, 64, Conf(64, 8, 16, 8, 16, 1), "matrix", 4),  # as many as fit
+    (9400, 64, Conf(64, 8, 16, 8, 16, 1), "staged", None),
+    (9650, 64, Conf(64, 8, 8, 8, 16, 1), "staged", None),
+    (9750, 64, None, "staged", None),
+]
+
+
+@pytest.mark.parametrize("case", ROWS_PER_BARRIER, ids=lambda c: "-".join(str(v) for v in (
+    *c[:2], "default" if c[2] is None else (c[2].threads_d1, c[2].items_d0, c[2].items_d1, c[2].unroll))).replace(" ", ""))
+def test_rows_per_barrier(torch_cuda, case):
+    channels, dms, conf, form, rows = case
+    job = beam(channels, 300, dms, 0.1, (3,))
+    if conf is not None:
+        job["plan"].set_conf(DD_SINGLE_STEP, conf)
+    info = job["plan"].launch_info(DD_SINGLE_STEP)
+    assert info["form"] == form and (info["rows_per_barrier"] == rows if rows else info["rows_per_barrier"] >= 4), info
+    job["plan"].dedisperse(job["input"].data_ptr(), job["out"].data_ptr(), stream=stream_of(torch_cuda))
+    verify(job, f"{case}")
