@@ -563,8 +563,20 @@ void set_default_confs(dd_plan *p) {
     p->conf[m] = plain_conf(mode);
     if (mode != DD_SINGLE_STEP && !p->two_step) continue;
     Geometry plain, g;
-    const dd_conf c = default_conf(p, mode);
+    dd_conf c = default_conf(p, mode);
     if (geometry_of(p, mode, c, g) != DD_OK) continue;
+    // Row windows that the pipeline does not take are staged a group at a time, the
+    // more rows the better up to eight, and a tile of 512 samples or more wants them
+    // staged at all: float rows, us, with 8, 4 and 2 rows and through the caches, 1497
+    // DMs x 3626 samples of 314 channels 401, 573, 907 and 1458; 357 x 16741 of 23 channels
+    // (8 do not fit) 67, 107 and 119.  Tiles of 256 samples: 436, 702, 1215 and 354 (131 x 8415 of 534).
+    if (!g.staged && c.items_d0 >= 8) {
+      dd_conf rows = c;
+      for (rows.unroll = 8; rows.unroll > 1; rows.unroll /= 2)
+        if (geometry_of(p, mode, rows, g) == DD_OK && g.local) break;
+      if (geometry_of(p, mode, rows, g) == DD_OK && !g.staged && g.local) c = rows;
+      if (geometry_of(p, mode, c, g) != DD_OK) continue;
+    }
     const bool packed = mode != DD_STEP_TWO && p->input_bits < 8;
     if ((g.staged && !packed) || (geometry_of(p, mode, p->conf[m], plain) == DD_OK && g.staged >= plain.staged))
       p->conf[m] = c;

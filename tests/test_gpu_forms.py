@@ -264,3 +264,17 @@ def test_rows_per_barrier(torch_cuda, case):
     assert info["form"] == form and (info["rows_per_barrier"] == rows if rows else info["rows_per_barrier"] >= 4), info
     job["plan"].dedisperse(job["input"].data_ptr(), job["out"].data_ptr(), stream=stream_of(torch_cuda))
     verify(job, f"{case}")
+
+
+# channels, dms, samples, step, bits: plans whose row windows the pipeline cannot take in
+# the shape of their sizes, and the form that their own configuration runs
+WIDE_WINDOWS = [(73, 961, 15484, 6.13, 32, "groups"), (64, 500, 8000, 12.0, 32, "groups"),
+                (61, 53, 16745, 11.6, 32, "direct"), (73, 961, 15484, 0.2, 32, "staged")]
+
+
+@pytest.mark.parametrize("case", WIDE_WINDOWS, ids=lambda c: "-".join(map(str, c)))
+def test_default_shape_of_wide_windows(torch_cuda, case):
+    channels, dms, samples, step, bits, form = case
+    w = workloads.tiny(channels=channels, samples=samples, dms=dms, step=step, min_freq=1250.0, bandwidth=300.0 / channels)
+    plan = Plan(w.obs, 128, input_bits=bits)
+    assert plan.launch_info(DD_SINGLE_STEP)["form"] == form
