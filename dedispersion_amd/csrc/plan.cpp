@@ -458,14 +458,14 @@ void set_byte_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, ByteKerne
 
 namespace {
 
-dd_conf conf_of(uint32_t wavefronts, uint32_t items_d0, uint32_t items_d1, uint32_t unroll) {
+dd_conf conf_of(uint32_t wavefronts, uint32_t items_d0, uint32_t items_d1, uint32_t unroll, uint32_t local = 1) {
   dd_conf c{};
   c.threads_d0 = 64;
   c.threads_d1 = wavefronts;
   c.items_d0 = items_d0;
   c.items_d1 = items_d1;
   c.unroll = unroll;
-  c.local = 1;
+  c.local = local;
   return c;
 }
 
@@ -514,17 +514,34 @@ dd_conf default_conf(const dd_plan *p, dd_mode mode) {
   const uint32_t cus = p->compute_units;
   const bool floats = p->input_bits == 32;
   if (mode == DD_STEP_TWO) {
-    // few rows (subbands) and much output: small groups of rows and many
-    // workgroups per compute unit, once there are several for each (both steps, us,
-    // at 16, 32, 64 and 128 coarse x 32 fine DMs and 256, 768, 3072 and 8192 tiles of
-    // 512 samples x 32 DMs: four wavefronts of 8 DMs and 2 rows per barrier 43, 60.5,
-    // 202 and 478; eight wavefronts of 4 DMs and 8 rows 36.5, 69, 245 and 619)
-    const uint32_t d1 = o.nr_dms <= 16 ? 2 : o.nr_dms <= 32 ? 4 : 8;
-    const uint64_t tiles = (uint64_t)((z.nr_samples + 511) / 512) * ((o.nr_dms + 8 * d1 - 1) / (8 * d1)) *
-                           o.nr_synthesized_beams * o.nr_dms_subbanding;
-    if (tiles >= 2ull * cus && d1 == 4) return conf_of(4, 8, 8, 2);
-    if (tiles >= 4ull * cus) return conf_of(8, 8, d1, 2);
-    return conf_of(8, tiles >= (uint64_t)cus * 3 / 4 ? 8 : 4, d1, 8);
+    auto tiles = [&](uint32_t dms_per_tile) {  // of 512 samples
+      return (uint64_t)((z.nr_samples + 511) / 512) * ((o.nr_dms + dms_per_tile - 1) / dms_per_tile) *
+             o.nr_synthesized_beams * o.nr_dms_subbanding;
+    };
+    // Few rows (subbands) are one group or two: a pipeline has nothing to run ahead of,
+    // and its four copies of every row are not read often enough.  Staged once, in the
+    // largest tile that still fills the device.  Measured over 420 plans of 1-64
+    // subbands, 1-128 coarse and 1-96 fine DMs and 256-24576 samples, us in one group and
+    // pipelined: 1 subband, 119 x 29 DMs x 7561 16.7 and 21.9; 8, 103 x 10 x 1093 6.0 and
+    // 9.0; 16, 50 x 10 x 2567 9.1 and 11.6; 32, 22 x 19 x 282 10.0 and 9.2.
+    if (o.nr_subbands <= 16) {
+      const uint32_t d1 = o.nr_dms <= 8 ? 1 : 2;
+      if (o.nr_dms > 16 && tiles(32) >= 2ull * cus) return conf_of(8, 8, 4, 8, 2);
+      return conf_of(8, 2 * tiles(8 * d1) >= cus ? 8 : 4, d1, 8, 2);
+    }
+    // Much output: small groups of rows and many workgroups per compute unit, once
+    // there are several for each (both steps, us, at 16, 32, 64 and 128 coarse x 32 fine
+    // DMs and 256, 768, 3072 and 8192 tiles of 512 samples x 32 DMs: four wavefronts of 8
+    // DMs and 2 rows per barrier 43, 60.5, 202 and 478; eight wavefronts of 4 DMs and 8
+    // rows 36.5, 69, 245 and 619).  64 DMs per tile only where there are about as many
+    // for each of several workgroups, or one tile instead of two (32 subbands, 38 DMs
+    // 14.9 and 17.4; 64 subbands, 45 DMs 22.7 and 15.5, 83 DMs x 1055 65.9 and 48.4).
+    if (o.nr_dms > 40 && tiles(64) >= 4ull * cus) return conf_of(8, 8, 8, 2);
+    const uint32_t d1 = o.nr_dms <= 16 ? 2 : o.nr_dms <= 32 || o.nr_dms > 40 ? 4 : 8;
+    const uint64_t n = tiles(8 * d1);
+    if (n >= 2ull * cus && d1 == 4) return conf_of(4, 8, 8, 2);
+    if (n >= 4ull * cus) return conf_of(8, 8, d1, 2);
+    return conf_of(8, n >= (uint64_t)cus * 3 / 4 ? 8 : 4, d1, 8);
   }
   const bool single = mode == DD_SINGLE_STEP;
   const uint32_t rows = single ? o.nr_channels : cps(p), dms = single ? o.nr_dms : o.nr_dms_subbanding;
@@ -550,7 +567,7 @@ dd_conf plain_conf(dd_mode mode) {
   switch (mode) {
   case DD_SINGLE_STEP: return conf_of(8, 16, 8, 4);
   case DD_STEP_ONE: return conf_of(4, 16, 8, 4);
-  default: return conf_of(8, 8, 4, 8);
+  default: return conf_of(8, 8, 4, 8, 2);
   }
 }
 
@@ -570,7 +587,7 @@ void set_default_confs(dd_plan *p) {
     // staged at all: float rows, us, with 8, 4 and 2 rows and through the caches, 1497
     // DMs x 3626 samples of 314 channels 401, 573, 907 and 1458; 357 x 16741 of 23 channels
     // (8 do not fit) 67, 107 and 119.  Tiles of 256 samples: 436, 702, 1215 and 354 (131 x 8415 of 534).
-    if (!g.staged && c.items_d0 >= 8) {
+    if (!g.staged && (c.local == 1 || !g.local) && c.items_d0 >= 8) {
       dd_conf rows = c;
       for (rows.unroll = 8; rows.unroll > 1; rows.unroll /= 2)
         if (geometry_of(p, mode, rows, g) == DD_OK && g.local) break;

@@ -278,3 +278,25 @@ def test_default_shape_of_wide_windows(torch_cuda, case):
     w = workloads.tiny(channels=channels, samples=samples, dms=dms, step=step, min_freq=1250.0, bandwidth=300.0 / channels)
     plan = Plan(w.obs, 128, input_bits=bits)
     assert plan.launch_info(DD_SINGLE_STEP)["form"] == form
+
+
+# subbands, coarse DMs, fine DMs, samples, the default's form and tile (samples per lane, DMs
+# per wavefront): one group of rows up to 16 subbands, more go through the pipeline
+DEFAULT_STEP_TWO = [
+    (1, 3, 7, 700, "groups", 4, 1), (2, 40, 8, 2300, "groups", 8, 1), (3, 2, 9, 1100, "groups", 4, 2),
+    (16, 30, 16, 2600, "groups", 8, 2), (16, 2, 33, 520, "groups", 4, 2), (4, 260, 17, 900, "groups", 8, 4),
+    (17, 2, 9, 700, "staged", 4, 2), (17, 3, 33, 700, "staged", 4, 8), (18, 2, 41, 700, "staged", 4, 4),
+    (17, 180, 45, 1300, "staged", 8, 8), (20, 530, 41, 500, "staged", 8, 8),
+]
+
+
+@pytest.mark.parametrize("case", DEFAULT_STEP_TWO, ids=lambda c: "-".join(map(str, c)))
+def test_default_shape_of_step_two(torch_cuda, case):
+    subbands, coarse, fine, samples, form, items_d0, items_d1 = case
+    job = beam(subbands * 2, samples, fine, 0.4, subbands=subbands, coarse=coarse, coarse_step=0.1)
+    plan = job["plan"]
+    conf = plan.get_conf(DD_STEP_TWO)
+    assert plan.launch_info(DD_STEP_TWO)["form"] == form and (conf.items_d0, conf.items_d1) == (items_d0, items_d1), conf
+    plan.step_one(job["input"].data_ptr(), job["mid"].data_ptr(), stream=stream_of(torch_cuda))
+    plan.step_two(job["mid"].data_ptr(), job["out"].data_ptr(), stream=stream_of(torch_cuda))
+    verify(job, f"{case}")
