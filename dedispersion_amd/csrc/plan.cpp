@@ -557,7 +557,17 @@ dd_conf default_conf(const dd_plan *p, dd_mode mode) {
     return c;
   }
   if (floats) return dms > 32 ? conf_of(8, 8, 8, 2) : dms > 16 ? conf_of(8, 8, 4, 2) : conf_of(8, 8, 2, 4);
-  return dms > 64 ? conf_of(8, 16, 8, 4) : dms > 16 ? conf_of(8, 8, 4, 8) : conf_of(8, 8, 2, 8);
+  // Byte rows.  The largest tiles once there are several for each compute unit, of 64 DMs
+  // where the last is at least half full; and larger ones for a few rows and DMs in a
+  // large grid, which is bound by its outputs (us: 62 rows, 89 DMs x 2746 x 8 subbands
+  // 33.9 in 64 DMs x 1024 samples, 16.2 in 32 x 512; 40 rows, 68 x 9521 x 128 164 in 64 DMs,
+  // 151 in 32; 3 rows, 2 x 7905 x 128 9.4 in 16 x 512, 6.2 in 16 x 1024).
+  auto tiles = [&](uint32_t samples_per_tile, uint32_t dms_per_tile) {
+    return (uint64_t)((samples + samples_per_tile - 1) / samples_per_tile) * ((dms + dms_per_tile - 1) / dms_per_tile) * slices;
+  };
+  if (dms > 64 && tiles(1024, 64) >= 4ull * cus) return roundup(dms, 64) - dms < 32 ? conf_of(8, 16, 8, 4) : conf_of(4, 16, 8, 4);
+  if (dms > 16) return rows <= 4 && tiles(512, 32) >= 16ull * cus ? conf_of(4, 16, 8, 4) : conf_of(8, 8, 4, 8);
+  return rows <= 4 && tiles(512, 16) >= 4ull * cus ? conf_of(4, 16, 4, 4) : conf_of(8, 8, 2, 8);
 }
 
 // The shapes that every plan started from.  What they refuse (row windows too

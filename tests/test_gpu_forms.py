@@ -300,3 +300,23 @@ def test_default_shape_of_step_two(torch_cuda, case):
     plan.step_one(job["input"].data_ptr(), job["mid"].data_ptr(), stream=stream_of(torch_cuda))
     plan.step_two(job["mid"].data_ptr(), job["out"].data_ptr(), stream=stream_of(torch_cuda))
     verify(job, f"{case}")
+
+
+# channels per subband, subbands, coarse DMs, samples, the default's tile: wavefronts, samples
+# per lane, DMs per wavefront
+DEFAULT_STEP_ONE = [
+    (3, 128, 2, 7905, 4, 16, 4), (3, 16, 2, 7905, 8, 8, 2), (5, 128, 2, 7905, 8, 8, 2), (4, 128, 33, 8300, 4, 16, 8),
+    (8, 8, 89, 2746, 8, 8, 4), (5, 128, 68, 9521, 4, 16, 8), (5, 128, 96, 4200, 4, 16, 8), (5, 128, 97, 4200, 8, 16, 8),
+]
+
+
+@pytest.mark.parametrize("case", DEFAULT_STEP_ONE, ids=lambda c: "-".join(map(str, c)))
+def test_default_shape_of_step_one(torch_cuda, case):
+    per, subbands, coarse, samples, waves, items_d0, items_d1 = case
+    job = beam(subbands * per, samples, 1, 0.0, subbands=subbands, coarse=coarse, coarse_step=0.1)
+    plan = job["plan"]
+    conf = plan.get_conf(DD_STEP_ONE)
+    assert (conf.threads_d1, conf.items_d0, conf.items_d1) == (waves, items_d0, items_d1), conf
+    plan.step_one(job["input"].data_ptr(), job["mid"].data_ptr(), stream=stream_of(torch_cuda))
+    plan.step_two(job["mid"].data_ptr(), job["out"].data_ptr(), stream=stream_of(torch_cuda))
+    verify(job, f"{case}")
