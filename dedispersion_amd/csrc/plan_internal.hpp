@@ -49,10 +49,11 @@ struct ShiftTable {
   DeviceBuffer<uint32_t> dev;
   std::vector<uint32_t> host;
   uint32_t at(uint32_t r, uint32_t d) const { return host[(size_t)r * pitch + d]; }
+  // Shifts grow with the DM (its step is never negative, and a negative product
+  // becomes 0), so the last DM holds every row's largest.
   uint32_t max_shift() const {
     uint32_t m = 0;
-    for (uint32_t r = 0; r < rows; ++r)
-      for (uint32_t d = 0; d < dms; ++d) m = std::max(m, at(r, d));
+    for (uint32_t r = 0; r < rows && dms > 0; ++r) m = std::max(m, at(r, dms - 1));
     return m;
   }
   // Largest shift spread inside any DM tile of `tile` consecutive DMs

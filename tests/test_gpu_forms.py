@@ -320,3 +320,23 @@ def test_default_shape_of_step_one(torch_cuda, case):
     plan.step_one(job["input"].data_ptr(), job["mid"].data_ptr(), stream=stream_of(torch_cuda))
     plan.step_two(job["mid"].data_ptr(), job["out"].data_ptr(), stream=stream_of(torch_cuda))
     verify(job, f"{case}")
+
+
+@pytest.mark.parametrize("tables", ["formula", "rising", "zero"])
+@pytest.mark.parametrize("first,step", [(0.0, 0.7), (40.0, 0.3), (3.0, 0.0)])
+def test_largest_shift(torch_cuda, tables, first, step):
+    """The sizes' largest shifts are those of the integer tables, also where step one's
+    delays relative to a subband's top channel are negative (a table that rises)."""
+    w = workloads.tiny(channels=24, samples=100, dms=9, step=step, first=first, subbands=4, coarse=7, coarse_step=2.5,
+                       coarse_first=first)
+    plan = Plan(w.obs, 128)
+    if tables != "formula":
+        a, b = plan.get_shifts()
+        a[:24] = np.linspace(0.1, 3.0, 24) if tables == "rising" else 0.0
+        b[:4] = np.linspace(0.1, 3.0, 4) if tables == "rising" else 0.0
+        plan.set_shifts(a, b)
+    z = plan.sizes
+    for mode, largest in ((DD_SINGLE_STEP, z.max_shift), (DD_STEP_ONE, z.max_shift_step_one), (DD_STEP_TWO, z.max_shift_step_two)):
+        table = plan.get_integer_shifts(mode)
+        assert largest == table.max()
+        assert np.all(np.diff(table.astype(np.int64), axis=1) >= 0)
