@@ -110,7 +110,7 @@ FORMS = ("direct", "groups", "staged", "patterns", "matrix", "pairs", "whole")
 
 def _launch_dict(i) -> dict:
     return {"form": FORMS[i.form], "rows_per_barrier": i.rows_per_barrier, "lds_bytes": i.lds_bytes,
-            "many_windows": bool(i.many_windows), "tiles_per_run": i.tiles_per_run}
+            "many_windows": bool(i.many_windows), "copies": i.copies, "tiles_per_run": i.tiles_per_run}
 
 
 class Plan:

@@ -131,6 +131,7 @@ class DDLaunchInfo(ctypes.Structure):
         ("rows_per_barrier", c_uint32),
         ("lds_bytes", c_uint32),
         ("many_windows", c_uint32),
+        ("copies", c_uint32),
         ("tiles_per_run", c_uint32),
     ]
 

@@ -164,8 +164,8 @@ template <typename L> void merge_geometry(KindQueue &k, const L &launch, bool fi
 // Every job's launches under the batch configuration (and its plan's own),
 // sorted into the kind queues or beside them; `pairs`: prepare the compact
 // step two's paired kernel where a job allows it; `single`, `one`: the form
-// of the byte kernel of the single-step and step-one jobs.
-dd_status plan_jobs(dd_batch *b, bool pairs, bool whole, ByteKernel single, ByteKernel one) {
+// of the byte kernel of the single-step and step-one jobs; `two`: that of the float step two.
+dd_status plan_jobs(dd_batch *b, bool pairs, bool whole, ByteKernel single, ByteKernel one, FloatKernel two) {
   for (auto &k : b->q) {
     k.u8.clear();
     k.f32.clear();
@@ -225,7 +225,7 @@ dd_status plan_jobs(dd_batch *b, bool pairs, bool whole, ByteKernel single, Byte
       F32Launch L2;
       s = prepare_step_one(job.plan, b->conf[DD_STEP_ONE], job.in, job.mid, L1, one);
       if (s == DD_OK)
-        s = prepare_step_two(job.plan, b->conf[DD_STEP_TWO], job.mid, job.out, job.first_sbeam, job.nr_sbeams, L2);
+        s = prepare_step_two(job.plan, b->conf[DD_STEP_TWO], job.mid, job.out, job.first_sbeam, job.nr_sbeams, L2, two);
       // the plan's own launches prepared above; a batch configuration that
       // cannot run this job (its LDS, its windows) leaves it beside the batch
       if (s != DD_OK && s != DD_ERR_CONFIGURATION) return s;
@@ -240,7 +240,8 @@ dd_status plan_jobs(dd_batch *b, bool pairs, bool whole, ByteKernel single, Byte
         if (s == DD_ERR_CONFIGURATION) fits = false;
         else if (s != DD_OK) return s;
       } else if (fits) {
-        fits = staged(L2);
+        // one kernel for the batch: jobs whose row lists leave no room for one copy run beside it
+        fits = staged(L2) && (two != FloatKernel::kOneCopy || L2.g.narrow);
       }
       b->beside.push_back(!fits);
       b->compact_job.push_back(fits && b->compact);
@@ -268,6 +269,24 @@ ByteKernel common_byte_kernel(const KindQueue &k) {
   for (const U8Launch &L : k.u8) tiles[L.g.matrix ? 1 : 0] += L.k.n_tiles;
   if (tiles[0] == 0 || tiles[1] == 0) return ByteKernel::kByRule;
   return tiles[1] >= tiles[0] ? ByteKernel::kMatrix : ByteKernel::kVector;
+}
+
+// Likewise of the float step two: the form for the batch's tiles together.
+FloatKernel common_float_kernel(const dd_batch *b) {
+  if (b->compact) return FloatKernel::kByRule;
+  uint64_t tiles = 0;
+  bool staged_jobs[2] = {false, false};
+  const dd_plan *plan = nullptr;
+  for (const Job &job : b->jobs)
+    if (job.kind == kTwoStep) plan = job.plan;
+  if (!plan) return FloatKernel::kByRule;
+  for (const F32Launch &L : b->q[DD_STEP_TWO].f32) {
+    tiles += L.k.n_tiles;
+    staged_jobs[L.g.narrow ? 1 : 0] = true;
+  }
+  const bool narrow = one_copy_is_faster(plan, b->conf[DD_STEP_TWO], tiles);
+  if (!staged_jobs[narrow ? 0 : 1]) return FloatKernel::kByRule;  // they agree
+  return narrow ? FloatKernel::kOneCopy : FloatKernel::kFourCopies;
 }
 
 // Joins sample tiles of the uint16 step two into runs that one workgroup sums one
@@ -315,7 +334,7 @@ dd_status plan_batch(dd_batch *b, std::vector<TileDesc> (&tiles_of)[3]) {
   // one step-two kernel for the whole batch: the paired one only when every
   // job in the batch kernels took it
   const bool pairs = b->compact && b->paired_requested;
-  dd_status st = plan_jobs(b, pairs, true, ByteKernel::kByRule, ByteKernel::kByRule);
+  dd_status st = plan_jobs(b, pairs, true, ByteKernel::kByRule, ByteKernel::kByRule, FloatKernel::kByRule);
   if (st != DD_OK) return st;
   bool all = true;
   bool whole = true;  // likewise
@@ -324,8 +343,9 @@ dd_status plan_batch(dd_batch *b, std::vector<TileDesc> (&tiles_of)[3]) {
     whole = whole && L.g.whole;
   }
   ByteKernel single = common_byte_kernel(b->q[DD_SINGLE_STEP]), one = common_byte_kernel(b->q[DD_STEP_ONE]);
-  if ((pairs && !all) || (b->compact && !pairs && !whole) || single != ByteKernel::kByRule || one != ByteKernel::kByRule) {
-    st = plan_jobs(b, pairs && all, whole, single, one);
+  FloatKernel two = common_float_kernel(b);
+  if ((pairs && !all) || (b->compact && !pairs && !whole) || two != FloatKernel::kByRule || single != ByteKernel::kByRule || one != ByteKernel::kByRule) {
+    st = plan_jobs(b, pairs && all, whole, single, one, two);
     if (st != DD_OK) return st;
   }
   // a job that the matrix form has no room for (its row window) takes the others with it
@@ -334,7 +354,7 @@ dd_status plan_batch(dd_batch *b, std::vector<TileDesc> (&tiles_of)[3]) {
   if (mixed_single || mixed_one) {
     if (mixed_single) single = ByteKernel::kVector;
     if (mixed_one) one = ByteKernel::kVector;
-    st = plan_jobs(b, pairs && all, whole, single, one);
+    st = plan_jobs(b, pairs && all, whole, single, one, two);
     if (st != DD_OK) return st;
   }
   if (b->compact && b->q[DD_STEP_TWO].g.whole) run_tiles(b->q[DD_STEP_TWO], (uint32_t)b->cus);
@@ -350,8 +370,8 @@ dd_status plan_batch(dd_batch *b, std::vector<TileDesc> (&tiles_of)[3]) {
     if (tiles.size() > 0xFFFFFFF0u) return fail(DD_ERR_UNSUPPORTED, "too many tiles in one batch");
     k.n_tiles = (uint32_t)tiles.size();
     if (k.n_tiles == 0) continue;
-    // the persistent kernels also hold 16 bytes of static LDS (the claim slot, aligned)
-    if (k.g.lds_bytes + 16 > b->jobs.front().plan->max_lds || b->lds_reserve[m] > b->jobs.front().plan->max_lds)
+    // the persistent kernels also hold the claim slot
+    if (k.g.lds_bytes + kClaimSlot > b->jobs.front().plan->max_lds || b->lds_reserve[m] > b->jobs.front().plan->max_lds)
       return fail(DD_ERR_CONFIGURATION, "batch LDS demand exceeds the device limit");
     int per_cu = 0;
     if (m == DD_STEP_TWO) {

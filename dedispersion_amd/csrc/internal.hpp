@@ -156,6 +156,7 @@ struct Geometry {
   uint32_t wide;       // 1 = ... whose rows may take more than one window
   uint32_t whole;      // 1 = the uint16 step two with a tile's rows whole in LDS (kernels_u16_whole.hip)
   uint32_t many;       // 1 = the staged float kernel for slices of more than kF32Rows rows
+  uint32_t narrow;     // 1 = the staged float kernel with one copy of a row (kernels_f32_narrow.hip)
 };
 
 // Launchers (kernels_u8.hip / kernels_f32.hip).  Return hipSuccess or the
@@ -208,6 +209,13 @@ hipError_t launch_rowsum_f32_list(const RowSumF32Params *d_jobs, const TileDesc 
 hipError_t launch_rowsum_u16_list(const RowSumF32Params *d_jobs, const TileDesc *d_tiles, uint32_t n,
                                   const Geometry &g, hipStream_t stream);
 hipError_t rowsum_f32_batch_occupancy(const Geometry &g, int *per_cu);
+// The same with one copy of a row (kernels_f32_narrow.hip; Geometry::narrow).
+hipError_t launch_rowsum_f32_narrow(const RowSumF32Params &p, const Geometry &g, hipStream_t stream);
+hipError_t launch_rowsum_f32_narrow_batch(const RowSumF32Params *d_jobs, const TileQueues &q, const Geometry &g,
+                                          uint32_t workgroups, hipStream_t stream);
+hipError_t launch_rowsum_f32_narrow_list(const RowSumF32Params *d_jobs, const TileDesc *d_tiles, uint32_t n,
+                                         const Geometry &g, hipStream_t stream);
+hipError_t rowsum_f32_narrow_batch_occupancy(const Geometry &g, int *per_cu);
 hipError_t launch_clear_words(uint32_t *d_words, uint32_t n, hipStream_t stream);
 // Step two over uint16 step-one sums (kernels_u16_staged.hip): the staged
 // pipeline with a window of g.win uint16 elements per row, four copies per
@@ -240,6 +248,7 @@ hipError_t launch_rowsum_u8_matrix_list(const RowSumU8Params *d_jobs, const Tile
 hipError_t rowsum_u8_matrix_batch_occupancy(const Geometry &g, int *per_cu);
 constexpr uint32_t kU8MatrixReach = 32;     // bytes that its operands reach past a row's window
 constexpr uint32_t kU8MatrixWindow = 2048;  // widest row window that it stages (two loads per wavefront)
+constexpr uint32_t kClaimSlot = 16;          // static LDS of the persistent kernels (the claim slot, aligned)
 constexpr uint32_t kStagedSlotsPerWave = 2;  // rows staged per wavefront per group
 constexpr uint32_t kU8StagedChunks = 2;      // 16-byte staging loads per lane per row (window <= 2 KiB)
 inline uint32_t f32_staged_chunks(uint32_t run) { return run / 4 + 1; }

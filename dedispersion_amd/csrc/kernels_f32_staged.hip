@@ -18,6 +18,8 @@
 //    wavefront that stages it, and published through LDS as byte addresses.
 //  * Workgroups are ordered XCD-aware (staged_common.hpp).
 //
+// Tiles of few DMs in large grids run kernels_f32_narrow.hip, one copy of a row.
+//
 // Bound by the LDS reads, 4 bytes per addition, at 16 bytes per lane.  Measured on
 // MI355X against one copy per row read 4 bytes at a time (us, one to the other, the
 // same inputs and tile shape; then each at its best shape): 768 channels x 512 DMs x
@@ -273,6 +275,7 @@ template <typename F> hipError_t dispatch(const Geometry &g, F &&shaped) {
 } // namespace
 
 hipError_t launch_rowsum_f32_staged(const RowSumF32Params &p, const Geometry &g, hipStream_t stream) {
+  if (g.narrow) return launch_rowsum_f32_narrow(p, g, stream);
   return dispatch(g, [&](auto run, auto dpw, auto many) {
     hipLaunchKernelGGL((rowsum_f32_staged<run.value, dpw.value, many.value>), dim3(p.n_tiles), dim3(64 * g.threads_d1),
                        g.lds_bytes, stream, p);
@@ -282,6 +285,7 @@ hipError_t launch_rowsum_f32_staged(const RowSumF32Params &p, const Geometry &g,
 
 hipError_t launch_rowsum_f32_batch(const RowSumF32Params *d_jobs, const TileQueues &q, const Geometry &g,
                                    uint32_t workgroups, hipStream_t stream) {
+  if (g.narrow) return launch_rowsum_f32_narrow_batch(d_jobs, q, g, workgroups, stream);
   return dispatch(g, [&](auto run, auto dpw, auto many) {
     hipLaunchKernelGGL((rowsum_f32_batch<run.value, dpw.value, many.value>), dim3(workgroups), dim3(64 * g.threads_d1),
                        g.lds_bytes, stream, d_jobs, q);
@@ -291,6 +295,7 @@ hipError_t launch_rowsum_f32_batch(const RowSumF32Params *d_jobs, const TileQueu
 
 hipError_t launch_rowsum_f32_list(const RowSumF32Params *d_jobs, const TileDesc *d_tiles, uint32_t n, const Geometry &g,
                                   hipStream_t stream) {
+  if (g.narrow) return launch_rowsum_f32_narrow_list(d_jobs, d_tiles, n, g, stream);
   return dispatch(g, [&](auto run, auto dpw, auto many) {
     hipLaunchKernelGGL((rowsum_f32_list<run.value, dpw.value, many.value>), dim3(n), dim3(64 * g.threads_d1), g.lds_bytes, stream,
                        d_jobs, d_tiles, n);
@@ -299,6 +304,7 @@ hipError_t launch_rowsum_f32_list(const RowSumF32Params *d_jobs, const TileDesc 
 }
 
 hipError_t rowsum_f32_batch_occupancy(const Geometry &g, int *per_cu) {
+  if (g.narrow) return rowsum_f32_narrow_batch_occupancy(g, per_cu);
   return dispatch(g, [&](auto run, auto dpw, auto many) {
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, rowsum_f32_batch<run.value, dpw.value, many.value>,
                                                         (int)(64 * g.threads_d1), (size_t)g.lds_bytes);

@@ -268,6 +268,17 @@ uint64_t float_tiles(const dd_plan *p, dd_mode mode, uint32_t samples_per_tile, 
 
 } // namespace
 
+// A row's DMs have to pay for its four copies, and their LDS and loads count where
+// workgroups share the compute units.  Time of four copies in that of one, over 1008
+// shapes and launches (the single step over 40 to 1536 channels, 64 to 1024 DMs and 4096
+// to 24576 samples, step two of 32 subbands): up to 4 wavefronts per compute unit in all
+// 0.30-1.57, mean 0.64; more, and tiles of 32 DMs or of 128 sums per lane and wavefront row
+// 0.31-1.54, mean 0.74; the rest 0.45-3.1, mean 1.42.  The rule is 2% from the better of both.
+bool one_copy_is_faster(const dd_plan *p, const dd_conf &c, uint64_t tiles) {
+  const uint32_t dms = c.threads_d1 * c.items_d1;
+  return dms < 32 && dms * c.items_d0 < 128 && tiles * c.threads_d1 > 4ull * p->compute_units;
+}
+
 dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry &g) {
   if (c.split_batches) return fail(DD_ERR_UNSUPPORTED, "split batches mode is not implemented");
   if (c.threads_d0 != 64) return fail(DD_ERR_CONFIGURATION, "threads_d0 must be 64 (one wavefront along samples)");
@@ -283,6 +294,7 @@ dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry
   g.matrix = 0;
   g.wide = 0;
   g.many = 0;
+  g.narrow = 0;
   g.whole = 0;
   g.unroll = c.unroll;
   // rows of floats: step two, and the single step and step one over float input
@@ -357,26 +369,7 @@ dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry
       g.win = roundup(ts + t.max_spread(tile), 4);
       g.lds_bytes = c.unroll * g.win * 4;
       if (stageable && g.win / 4 <= 64 * f32_staged_chunks(c.items_d0)) {
-        // [2 buffers][unroll rows][4 copies][win] | rows of a slice | DM addresses;
-        // rows staged per barrier are capped at what fits in LDS
-        const uint32_t slots = mode == DD_STEP_TWO ? p->obs.nr_subbands
-                               : mode == DD_SINGLE_STEP ? p->obs.nr_channels : cps(p);
-        auto lds_of = [&](uint32_t u) { return 4 * (4 * std::min(slots, kF32Rows) + 8 * u * g.win + 2 * u * tile); };
-        // A grid of more than one workgroup per compute unit leaves room for 16
-        // wavefronts on each, which the registers of all but the largest shapes
-        // allow (step two of 64 x 32 DMs x 24576 samples, eight wavefronts of 4 DMs:
-        // 8 rows per barrier and one workgroup 157 us, 4 rows and two 116).
-        const uint64_t tiles = float_tiles(p, mode, ts, tile);
-        const bool share = tiles > p->compute_units && c.items_d0 * c.items_d1 <= 64;
-        const uint64_t room = share ? std::min<uint64_t>(p->max_lds, (uint64_t)p->max_lds * c.threads_d1 / 16) : p->max_lds;
-        uint32_t unroll = c.unroll;
-        while (unroll > 1 && lds_of(unroll) > room) --unroll;
-        if (lds_of(unroll) <= p->max_lds) {
-          g.staged = 1;
-          g.many = slots > kF32Rows;
-          g.unroll = unroll;
-          g.lds_bytes = lds_of(unroll);
-        }
+        set_float_kernel(p, mode, c, FloatKernel::kByRule, g);
       }
     }
   } else {
@@ -425,6 +418,39 @@ dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry
   if (g.lds_bytes > p->max_lds)
     return fail(DD_ERR_CONFIGURATION, "LDS demand " + std::to_string(g.lds_bytes) + " bytes exceeds the device limit");
   return DD_OK;
+}
+
+void set_float_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, FloatKernel kernel, Geometry &g) {
+  // four copies: [2 buffers][rows per barrier][4 copies][win] | rows of a slice | DM
+  // addresses; one: rows | [2 buffers][rows per barrier][win] | DM offsets.  Rows per
+  // barrier are capped at what fits in LDS, beside the claim slot of a batch's kernel
+  const uint32_t tile = c.threads_d1 * c.items_d1;
+  const uint32_t slots = mode == DD_STEP_TWO ? p->obs.nr_subbands : mode == DD_SINGLE_STEP ? p->obs.nr_channels : cps(p);
+  const uint64_t limit = p->max_lds - kClaimSlot, tiles = float_tiles(p, mode, 64 * c.items_d0, tile);
+  auto lds_of = [&](uint32_t u, bool narrow) -> uint64_t {
+    if (narrow) return 4 * ((uint64_t)roundup(2 * slots, 4) + 2 * u * g.win + 2 * u * tile);
+    return 4 * (4 * std::min(slots, kF32Rows) + 8 * u * g.win + 2 * u * tile);
+  };
+  const bool narrow = (kernel == FloatKernel::kOneCopy || (kernel == FloatKernel::kByRule && one_copy_is_faster(p, c, tiles))) &&
+                      c.items_d0 * c.items_d1 < 128 && lds_of(1, true) <= limit;
+  uint32_t unroll = std::min(c.unroll, kStagedSlotsPerWave * c.threads_d1);
+  while (unroll > 1 && lds_of(unroll, narrow) > limit) --unroll;
+  if (lds_of(unroll, narrow) > limit) return;
+  // A grid of more than one workgroup per compute unit leaves room for 16
+  // wavefronts on each, which the registers of all but the largest shapes
+  // allow (step two of 64 x 32 DMs x 24576 samples, eight wavefronts of 4 DMs:
+  // 8 rows per barrier and one workgroup 157 us, 4 rows and two 127).  Also where
+  // the row list leaves room for less than that: 1536 channels, 1024 DMs x 12288,
+  // two wavefronts of 8 DMs x 512, 1 row 2479, 2 rows 2706, 4 rows 4099; four 1362,
+  // 1773 and 2087; two of 4 DMs 4256, 4269 and 6192.
+  const uint64_t room = p->max_lds * c.threads_d1 / 16;
+  if (!narrow && tiles > p->compute_units && c.items_d0 * c.items_d1 <= 64)
+    while (unroll > 1 && lds_of(unroll, narrow) > room) --unroll;
+  g.staged = 1;
+  g.narrow = narrow;
+  g.many = !narrow && slots > kF32Rows;
+  g.unroll = unroll;
+  g.lds_bytes = (uint32_t)lds_of(unroll, narrow);
 }
 
 void set_byte_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, ByteKernel kernel, Geometry &g) {
@@ -729,7 +755,7 @@ dd_status prepare_step_one(dd_plan *plan, const dd_conf &c, const uint8_t *d_inp
 }
 
 dd_status prepare_step_two(dd_plan *plan, const dd_conf &c, const float *d_intermediate, float *d_output,
-                           uint32_t first_sbeam, uint32_t nr_sbeams, F32Launch &L) {
+                           uint32_t first_sbeam, uint32_t nr_sbeams, F32Launch &L, FloatKernel kernel) {
   if (!plan || !d_intermediate || !d_output) return fail(DD_ERR_INVALID_ARGUMENT, "null argument");
   if (!plan->two_step) return fail(DD_ERR_INVALID_ARGUMENT, "plan has no subband path");
   const dd_observation &o = plan->obs;
@@ -741,6 +767,7 @@ dd_status prepare_step_two(dd_plan *plan, const dd_conf &c, const float *d_inter
     return fail(DD_ERR_INVALID_ARGUMENT, "subbanded batch shorter than samples + largest shift");
   dd_status s = geometry_of(plan, DD_STEP_TWO, c, L.g);
   if (s != DD_OK) return s;
+  if (kernel != FloatKernel::kByRule && L.g.staged) set_float_kernel(plan, DD_STEP_TWO, c, kernel, L.g);
   RowSumF32Params &k = L.k;
   k = RowSumF32Params{};
   k.in = d_intermediate;
@@ -791,6 +818,7 @@ dd_status prepare_step_two_u16(dd_plan *plan, const dd_conf &c, const void *d_in
     return fail(DD_ERR_CONFIGURATION, "step-two shift spread too large for the uint16 window");
   L.g.win = win;
   L.g.staged = 1;
+  L.g.narrow = 0;
   // rows | [2 buffers][unroll rows][4 copies][win / 2 dwords] | DM addresses;
   // rows staged per barrier are capped at what fits in LDS
   auto lds_of = [&](uint32_t u) { return 4 * (roundup(2 * plan->obs.nr_subbands, 4) + 4 * u * win + 2 * u * tile); };
@@ -950,6 +978,7 @@ dd_launch_info info_of(const Geometry &g) {
   info.rows_per_barrier = g.unroll;
   info.lds_bytes = g.lds_bytes;
   info.many_windows = g.wide;
+  info.copies = info.form != DD_FORM_STAGED ? 0 : g.narrow ? 1 : 4;
   info.tiles_per_run = 1;
   return info;
 }

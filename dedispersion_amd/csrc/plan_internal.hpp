@@ -165,6 +165,14 @@ enum class ByteKernel { kByRule, kVector, kMatrix };
 // matrix form has no such shape) and the LDS that it needs.
 void set_byte_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, ByteKernel kernel, Geometry &g);
 
+// Which form of the staged float kernel a launch takes, likewise.
+enum class FloatKernel { kByRule, kOneCopy, kFourCopies };
+// Whether one copy of a row is faster under configuration c in a launch of `tiles` workgroups.
+bool one_copy_is_faster(const dd_plan *p, const dd_conf &c, uint64_t tiles);
+// Sets the form, the rows per barrier and the LDS of a float geometry whose window is
+// set; leaves one alone whose rows do not fit.
+void set_float_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, FloatKernel kernel, Geometry &g);
+
 // What dd_plan_get_launch_info and dd_batch_get_launch_info say of a geometry.
 dd_launch_info info_of(const Geometry &g);
 
@@ -190,7 +198,8 @@ dd_status prepare_single(dd_plan *plan, const dd_conf &c, const uint8_t *d_input
 dd_status prepare_step_one(dd_plan *plan, const dd_conf &c, const uint8_t *d_input, float *d_intermediate,
                            U8Launch &L, ByteKernel kernel = ByteKernel::kByRule);
 dd_status prepare_step_two(dd_plan *plan, const dd_conf &c, const float *d_intermediate, float *d_output,
-                           uint32_t first_sbeam, uint32_t nr_sbeams, F32Launch &L);
+                           uint32_t first_sbeam, uint32_t nr_sbeams, F32Launch &L,
+                           FloatKernel kernel = FloatKernel::kByRule);
 // Step two over the uint16 sums that step one writes with out_u16 (a batch
 // that owns its intermediate): the launch of prepare_step_two with `in` read
 // as uint16 elements.  Fails with DD_ERR_CONFIGURATION when c does not select

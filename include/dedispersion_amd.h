@@ -226,6 +226,7 @@ typedef struct dd_launch_info {
   uint32_t rows_per_barrier; /* rows staged per barrier: the configuration's unroll, or fewer */
   uint32_t lds_bytes;        /* dynamic LDS per workgroup */
   uint32_t many_windows;     /* matrix form: rows may take more than one window of 32 samples */
+  uint32_t copies;           /* staged form: copies of a row in LDS, 4 (every read aligned) or 1 */
   uint32_t tiles_per_run;    /* whole rows: sample tiles that a workgroup sums one after another, else 1 */
 } dd_launch_info;
 /* The launch of `mode` under `conf` (NULL: the plan's configuration), for input at

@@ -340,3 +340,66 @@ def test_largest_shift(torch_cuda, tables, first, step):
         table = plan.get_integer_shifts(mode)
         assert largest == table.max()
         assert np.all(np.diff(table.astype(np.int64), axis=1) >= 0)
+
+
+# float rows: channels, samples, dms, shape, copies of a row in LDS.  One copy where
+# workgroups of few DMs share the compute units, four elsewhere
+FLOAT_SINGLE = [
+    *[(37, 20001, 1000, Conf(64, *s, 1), 1) for s in ((1, 4, 1, 2), (1, 16, 4, 2), (2, 8, 4, 3), (4, 8, 2, 8), (2, 4, 8, 4),
+                                                      (8, 8, 1, 16), (4, 4, 4, 5), (8, 4, 2, 7), (1, 8, 8, 1))],
+    (37, 20001, 1000, Conf(64, 8, 16, 1, 4, 1), 4), (37, 20001, 1000, Conf(64, 1, 16, 8, 2, 1), 4),
+    (37, 20001, 1000, Conf(64, 4, 4, 8, 4, 1), 4),
+    (37, 3001, 70, Conf(64, 1, 4, 4, 2, 1), 4), (37, 3001, 70, Conf(64, 8, 8, 1, 4, 1), 4),
+]
+
+
+@pytest.mark.parametrize("padding", [0, 128])
+@pytest.mark.parametrize("case", FLOAT_SINGLE, ids=lambda c: "-".join(map(str, (*c[:3], c[3].threads_d1, c[3].items_d0,
+                                                                               c[3].items_d1, c[3].unroll))))
+def test_copies_of_float_rows(torch_cuda, case, padding):
+    """Additions in the oracle's order: no tolerance."""
+    torch = torch_cuda
+    channels, samples, dms, conf, copies = case
+    w = workloads.tiny(channels=channels, samples=samples, dms=dms, step=0.05, min_freq=1250.0, bandwidth=300.0 / channels,
+                       zapped=(0, 9), seed=13)
+    plan = Plan(w.obs, padding, input_bits=32)
+    flags = zapped_flags(plan, w.zapped)
+    plan.set_zapped_channels(flags)
+    plan.set_conf(DD_SINGLE_STEP, conf)
+    info = plan.launch_info(DD_SINGLE_STEP)
+    assert info["form"] == "staged" and info["copies"] == copies, info
+    z = plan.sizes
+    host = (np.random.default_rng(3).standard_normal(z.input_elements) * 100.0).astype(np.float32)
+    d_in = torch.from_numpy(host).cuda()
+    d_out = torch.full((z.output_elements,), -1.0, dtype=torch.float32, device="cuda")
+    plan.dedisperse_f32(d_in.data_ptr(), d_out.data_ptr(), stream=stream_of(torch))
+    want = oracle.Oracle(w.obs, padding, threads=host_threads(), input_bits=32).dedispersion(host, flags)
+    got = d_out.cpu().numpy().reshape(want.shape)
+    compare_rows(got, want, samples, f"{case}")
+    assert np.all(got[..., samples:] == -1.0)
+
+
+@pytest.mark.parametrize("chunks", [0, 2])
+@pytest.mark.parametrize("case", ["large", "small", "together large", "large and small"])
+def test_copies_of_a_batch(torch_cuda, case, chunks):
+    """One form for all jobs of a batch, by their tiles together."""
+    big = dict(channels=40, samples=4000, dms=9, step=0.3, subbands=5, coarse=90, coarse_step=0.2, zapped=(2,))
+    small = dict(big, samples=600, coarse=7)
+    jobs = {"large": [big], "small": [small], "together large": [dict(small, coarse=40 + k, seed=k) for k in range(9)],
+            "large and small": [small, big, dict(small, beams=2)]}[case]
+    jobs = [beam(**j) for j in jobs]
+    batch = Batch()
+    for j in jobs:
+        add(batch, j)
+    batch.set_compact_intermediate(False)
+    batch.set_pipeline(chunks)
+    batch.set_conf(DD_STEP_TWO, Conf(64, 2, 4, 2, 3, 1))
+    info = batch.launch_info(DD_STEP_TWO)
+    assert info["form"] == "staged" and info["copies"] == (4 if case == "small" else 1), info
+    assert batch.info()["solo_jobs"] == 0
+    for graph in (False, True):
+        for j in jobs:
+            j["out"].fill_(-1.0)
+        batch.run(use_graph=graph, stream=stream_of(torch_cuda))
+        for k, j in enumerate(jobs):
+            verify(j, f"{case}, chunks {chunks}, graph {graph}, job {k}")
