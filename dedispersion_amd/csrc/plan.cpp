@@ -272,11 +272,13 @@ uint64_t float_tiles(const dd_plan *p, dd_mode mode, uint32_t samples_per_tile, 
 // workgroups share the compute units.  Time of four copies in that of one, over 1008
 // shapes and launches (the single step over 40 to 1536 channels, 64 to 1024 DMs and 4096
 // to 24576 samples, step two of 32 subbands): up to 4 wavefronts per compute unit in all
-// 0.30-1.57, mean 0.64; more, and tiles of 32 DMs or of 128 sums per lane and wavefront row
-// 0.31-1.54, mean 0.74; the rest 0.45-3.1, mean 1.42.  The rule is 2% from the better of both.
+// 0.30-1.3, tiles of 32 DMs, or of 16 up to 4 workgroups per compute unit, or of 128 DMs x
+// samples per lane 0.31-1.54 (1 of 8 above 1.1); the rest 0.45-3.1, mean 1.4.  The rule is
+// 2% from the better of both.
 bool one_copy_is_faster(const dd_plan *p, const dd_conf &c, uint64_t tiles) {
   const uint32_t dms = c.threads_d1 * c.items_d1;
-  return dms < 32 && dms * c.items_d0 < 128 && tiles * c.threads_d1 > 4ull * p->compute_units;
+  return dms < 32 && dms * c.items_d0 < 128 && tiles * c.threads_d1 > 4ull * p->compute_units &&
+         (dms < 16 || tiles > 4ull * p->compute_units);
 }
 
 dd_status geometry_of(const dd_plan *p, dd_mode mode, const dd_conf &c, Geometry &g) {
