@@ -594,7 +594,14 @@ dd_conf default_conf(const dd_plan *p, dd_mode mode) {
     return (uint64_t)((samples + samples_per_tile - 1) / samples_per_tile) * ((dms + dms_per_tile - 1) / dms_per_tile) * slices;
   };
   if (dms > 64 && tiles(1024, 64) >= 4ull * cus) return roundup(dms, 64) - dms < 32 ? conf_of(8, 16, 8, 4) : conf_of(4, 16, 8, 4);
-  if (dms > 16) return rows <= 4 && tiles(512, 32) >= 16ull * cus ? conf_of(4, 16, 8, 4) : conf_of(8, 8, 4, 8);
+  if (dms > 16) {
+    // wide windows are most of a small tile's staging, once there are several for each
+    // compute unit (64 x 12288 of 48 rows x 32 at 64 pc/cc 63 us in 32 DMs x 1024, 89 in 32 x 512)
+    const uint32_t spread = (single ? p->ish_single : p->ish_one).max_spread(32);
+    if (tiles(512, 32) > 2ull * cus && spread >= 300 && 1024 + spread + 36 <= 16 * 64 * kU8StagedChunks)
+      return conf_of(8, 16, 4, 4);
+    return rows <= 4 && tiles(512, 32) >= 16ull * cus ? conf_of(4, 16, 8, 4) : conf_of(8, 8, 4, 8);
+  }
   return rows <= 4 && tiles(512, 16) >= 4ull * cus ? conf_of(4, 16, 4, 4) : conf_of(8, 8, 2, 8);
 }
 
@@ -620,16 +627,21 @@ void set_default_confs(dd_plan *p) {
     Geometry plain, g;
     dd_conf c = default_conf(p, mode);
     if (geometry_of(p, mode, c, g) != DD_OK) continue;
-    // Row windows that the pipeline does not take are staged a group at a time, the
-    // more rows the better up to eight, and a tile of 512 samples or more wants them
-    // staged at all: float rows, us, with 8, 4 and 2 rows and through the caches, 1497
-    // DMs x 3626 samples of 314 channels 401, 573, 907 and 1458; 357 x 16741 of 23 channels
-    // (8 do not fit) 67, 107 and 119.  Tiles of 256 samples: 436, 702, 1215 and 354 (131 x 8415 of 534).
-    if (!g.staged && (c.local == 1 || !g.local) && c.items_d0 >= 8) {
+    if (mode == DD_STEP_TWO && c.local == 1 && !g.staged) continue;  // the plain shape: 100 x 20 DMs x 12288, 32 subbands, 101 against 124 us
+    // Row windows that the pipeline does not take are staged a group at a time: of
+    // fewer DMs where their spread is most of a window (float rows, 101 x 8273 of 23
+    // channels per subband at 58 pc/cc, 64 DMs 193 us, 16 DMs 39), the more rows the better
+    // up to eight, and a tile of 512 samples or more wants them staged at all (us, with
+    // 8, 4 and 2 rows and through the caches, 1497 DMs x 3626 samples of 314 channels 401,
+    // 573, 907 and 1458; 357 x 16741 of 23 channels, where 8 do not fit, 67, 107 and 119).
+    // Tiles of 256 samples: 436, 702, 1215 and 354 (131 x 8415 of 534).
+    if (!g.staged && c.local == 1 && c.items_d0 >= 8) {
+      const ShiftTable &t = mode == DD_SINGLE_STEP ? p->ish_single : p->ish_one;
       dd_conf rows = c;
+      while (rows.items_d1 > 2 && t.max_spread(rows.threads_d1 * rows.items_d1) > 256 * rows.items_d0) rows.items_d1 /= 2;
       for (rows.unroll = 8; rows.unroll > 1; rows.unroll /= 2)
-        if (geometry_of(p, mode, rows, g) == DD_OK && g.local) break;
-      if (geometry_of(p, mode, rows, g) == DD_OK && !g.staged && g.local) c = rows;
+        if (geometry_of(p, mode, rows, g) == DD_OK && (g.staged || g.local)) break;
+      if (geometry_of(p, mode, rows, g) == DD_OK && (g.staged || g.local)) c = rows;
       if (geometry_of(p, mode, c, g) != DD_OK) continue;
     }
     const bool packed = mode != DD_STEP_TWO && p->input_bits < 8;

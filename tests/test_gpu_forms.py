@@ -403,3 +403,29 @@ def test_copies_of_a_batch(torch_cuda, case, chunks):
         batch.run(use_graph=graph, stream=stream_of(torch_cuda))
         for k, j in enumerate(jobs):
             verify(j, f"{case}, chunks {chunks}, graph {graph}, job {k}")
+
+
+# plans of wide windows: channels per subband, subbands, coarse DMs, samples, their step, and the default's tile
+WIDE_STEP_ONE = [(44, 32, 33, 9000, 60.0, 8, 16, 4), (44, 32, 33, 9000, 1.0, 8, 8, 4), (44, 32, 33, 2000, 60.0, 8, 8, 4),
+                 (44, 8, 33, 17000, 60.0, 8, 8, 2), (20, 4, 40, 9000, 60.0, 8, 8, 2)]
+
+
+@pytest.mark.parametrize("case", WIDE_STEP_ONE, ids=lambda c: "-".join(map(str, c)))
+def test_default_shape_of_wide_step_one(torch_cuda, case):
+    per, subbands, coarse, samples, step, waves, items_d0, items_d1 = case
+    job = beam(subbands * per, samples, 1, 0.0, subbands=subbands, coarse=coarse, coarse_step=step)
+    plan = job["plan"]
+    conf = plan.get_conf(DD_STEP_ONE)
+    assert (conf.threads_d1, conf.items_d0, conf.items_d1) == (waves, items_d0, items_d1), conf
+    plan.step_one(job["input"].data_ptr(), job["mid"].data_ptr(), stream=stream_of(torch_cuda))
+    plan.step_two(job["mid"].data_ptr(), job["out"].data_ptr(), stream=stream_of(torch_cuda))
+    verify(job, f"{case}")
+
+
+def test_default_shape_of_wide_step_two(torch_cuda):
+    """Windows that the pipeline does not take: the shape of one group."""
+    w = workloads.tiny(channels=64, samples=12288, dms=20, step=3.0, subbands=32, coarse=100, coarse_step=60.0,
+                       min_freq=1250.0, bandwidth=300.0 / 64)
+    plan = Plan(w.obs, 128)
+    conf = plan.get_conf(DD_STEP_TWO)
+    assert plan.launch_info(DD_STEP_TWO)["form"] == "groups" and (conf.threads_d1, conf.items_d0, conf.items_d1) == (8, 8, 4)
