@@ -73,6 +73,7 @@ struct dd_batch {
   dd_conf conf[3]{};
   bool compact_requested = true;
   bool compact = false;  // in effect after build()
+  bool conf_set[3] = {false, false, false};  // a caller's configuration (dd_batch_set_conf)
   bool paired_requested = false;  // the compact step two adds subbands in pairs when every job allows it
   bool built = false;
   // one ordinary launch per job (float intermediate): dd_batch_run_per_job
@@ -124,9 +125,12 @@ struct dd_batch {
 
 namespace {
 
-dd_conf batch_default_conf(dd_mode mode) {
-  // The fastest staged shapes of an exhaustive sweep of both kernel kinds over
-  // 40 uneven 1536-channel beams on MI355X.
+// The fastest staged shapes of an exhaustive sweep of both kernel kinds over
+// 40 uneven 1536-channel beams on MI355X.  `pairs`: for the paired step two, which
+// stages half as many pairs per barrier as the configuration's rows (three beams of 32,
+// 64, 128 and 256 subbands, us, 4 and 8 rows: 138 and 100, 249 and 169, 448 and 290, 852 and
+// 539; four wavefronts of 16 x 8 with 8 rows 156, 284, 299 and 554).
+dd_conf batch_default_conf(dd_mode mode, bool pairs) {
   dd_conf c{};
   c.threads_d0 = 64;
   c.split_batches = 0;
@@ -134,7 +138,7 @@ dd_conf batch_default_conf(dd_mode mode) {
   c.threads_d1 = mode == DD_STEP_TWO ? 8 : 4;
   c.items_d0 = mode == DD_STEP_TWO ? 8 : 16;
   c.items_d1 = mode == DD_STEP_TWO ? 4 : 8;
-  c.unroll = mode == DD_STEP_TWO ? 4 : 8;
+  c.unroll = mode == DD_STEP_TWO && !pairs ? 4 : 8;
   return c;
 }
 
@@ -166,6 +170,7 @@ template <typename L> void merge_geometry(KindQueue &k, const L &launch, bool fi
 // step two's paired kernel where a job allows it; `single`, `one`: the form
 // of the byte kernel of the single-step and step-one jobs; `two`: that of the float step two.
 dd_status plan_jobs(dd_batch *b, bool pairs, bool whole, ByteKernel single, ByteKernel one, FloatKernel two) {
+  if (!b->conf_set[DD_STEP_TWO]) b->conf[DD_STEP_TWO] = batch_default_conf(DD_STEP_TWO, pairs);
   for (auto &k : b->q) {
     k.u8.clear();
     k.f32.clear();
@@ -205,6 +210,7 @@ dd_status plan_jobs(dd_batch *b, bool pairs, bool whole, ByteKernel single, Byte
         b->solo_single.push_back(P);
         continue;
       }
+      L.matrix_time = matrix_time_of(job.plan, DD_SINGLE_STEP, b->conf[DD_SINGLE_STEP]);
       KindQueue &k = b->q[DD_SINGLE_STEP];
       merge_geometry(k, L, k.u8.empty());
       k.flush = k.flush || L.flush;
@@ -250,6 +256,7 @@ dd_status plan_jobs(dd_batch *b, bool pairs, bool whole, ByteKernel single, Byte
         b->solo_two.push_back(P2);
         continue;
       }
+      L1.matrix_time = matrix_time_of(job.plan, DD_STEP_ONE, b->conf[DD_STEP_ONE]);
       KindQueue &k1 = b->q[DD_STEP_ONE];
       merge_geometry(k1, L1, k1.u8.empty());
       k1.flush = k1.flush || L1.flush;
@@ -262,13 +269,19 @@ dd_status plan_jobs(dd_batch *b, bool pairs, bool whole, ByteKernel single, Byte
   return DD_OK;
 }
 
-// One kernel runs all jobs of a kind: where the plans' rules differ, the form
-// that holds most of the tiles (kByRule: they agree).
+// One kernel runs all jobs of a kind: where the plans' rules differ, the form that
+// is faster for them together (kByRule: they agree).
 ByteKernel common_byte_kernel(const KindQueue &k) {
-  uint64_t tiles[2] = {0, 0};
-  for (const U8Launch &L : k.u8) tiles[L.g.matrix ? 1 : 0] += L.k.n_tiles;
-  if (tiles[0] == 0 || tiles[1] == 0) return ByteKernel::kByRule;
-  return tiles[1] >= tiles[0] ? ByteKernel::kMatrix : ByteKernel::kVector;
+  bool forms[2] = {false, false};
+  double matrix = 0, vector = 0;
+  for (const U8Launch &L : k.u8) {
+    const double work = (double)L.k.n_tiles * L.k.live_pitch;
+    forms[L.g.matrix ? 1 : 0] = true;
+    matrix += work * L.matrix_time;
+    vector += work;
+  }
+  if (!forms[0] || !forms[1]) return ByteKernel::kByRule;
+  return matrix <= vector ? ByteKernel::kMatrix : ByteKernel::kVector;
 }
 
 // Likewise of the float step two: the form for the batch's tiles together.
@@ -331,31 +344,37 @@ dd_status plan_batch(dd_batch *b, std::vector<TileDesc> (&tiles_of)[3]) {
   b->compact = b->compact_requested;
   for (const Job &job : b->jobs)
     if (job.kind == kTwoStep && 255u * std::max(job.plan->max_live_sub, 1u) > 65535u) b->compact = false;
-  // one step-two kernel for the whole batch: the paired one only when every
-  // job in the batch kernels took it
-  const bool pairs = b->compact && b->paired_requested;
-  dd_status st = plan_jobs(b, pairs, true, ByteKernel::kByRule, ByteKernel::kByRule, FloatKernel::kByRule);
-  if (st != DD_OK) return st;
-  bool all = true;
-  bool whole = true;  // likewise
-  for (const F32Launch &L : b->q[DD_STEP_TWO].f32) {
-    all = all && L.g.pairs;
-    whole = whole && L.g.whole;
-  }
-  ByteKernel single = common_byte_kernel(b->q[DD_SINGLE_STEP]), one = common_byte_kernel(b->q[DD_STEP_ONE]);
-  FloatKernel two = common_float_kernel(b);
-  if ((pairs && !all) || (b->compact && !pairs && !whole) || two != FloatKernel::kByRule || single != ByteKernel::kByRule || one != ByteKernel::kByRule) {
-    st = plan_jobs(b, pairs && all, whole, single, one, two);
+  // One kernel per kind for the whole batch.  Planned by every job's own rule first,
+  // then again without a form that some job in the batch kernels did not take: the
+  // paired step two, whole rows, and the forms of the byte and float kernels.
+  bool pairs = b->compact && b->paired_requested, whole = !pairs;
+  ByteKernel single = ByteKernel::kByRule, one = ByteKernel::kByRule;
+  FloatKernel two = FloatKernel::kByRule;
+  for (;;) {
+    dd_status st = plan_jobs(b, pairs, whole, single, one, two);
     if (st != DD_OK) return st;
-  }
-  // a job that the matrix form has no room for (its row window) takes the others with it
-  const bool mixed_single = common_byte_kernel(b->q[DD_SINGLE_STEP]) != ByteKernel::kByRule;
-  const bool mixed_one = common_byte_kernel(b->q[DD_STEP_ONE]) != ByteKernel::kByRule;
-  if (mixed_single || mixed_one) {
-    if (mixed_single) single = ByteKernel::kVector;
-    if (mixed_one) one = ByteKernel::kVector;
-    st = plan_jobs(b, pairs && all, whole, single, one, two);
-    if (st != DD_OK) return st;
+    bool all_pairs = true, all_whole = true, again = false;
+    for (const F32Launch &L : b->q[DD_STEP_TWO].f32) {
+      all_pairs = all_pairs && L.g.pairs;
+      all_whole = all_whole && L.g.whole;
+    }
+    if (pairs && !all_pairs) {
+      pairs = false;
+      whole = again = true;
+    } else if (b->compact && whole && !all_whole) {
+      whole = false;
+      again = true;
+    }
+    // a job that the matrix form has no room for (its row window, its input off a
+    // dword) takes the others with it
+    for (auto [kernel, kind] : {std::pair(&single, DD_SINGLE_STEP), std::pair(&one, DD_STEP_ONE)}) {
+      const ByteKernel common = common_byte_kernel(b->q[kind]);
+      if (common == ByteKernel::kByRule) continue;
+      *kernel = *kernel == ByteKernel::kByRule ? common : ByteKernel::kVector;
+      again = true;
+    }
+    if (two == FloatKernel::kByRule && (two = common_float_kernel(b)) != FloatKernel::kByRule) again = true;
+    if (!again) break;
   }
   if (b->compact && b->q[DD_STEP_TWO].g.whole) run_tiles(b->q[DD_STEP_TWO], (uint32_t)b->cus);
   for (int m = 0; m < 3; ++m) {
@@ -638,7 +657,7 @@ extern "C" {
 dd_status dd_batch_create(dd_batch **batch) {
   if (!batch) return fail(DD_ERR_INVALID_ARGUMENT, "null argument");
   dd_batch *b = new dd_batch();
-  for (int m = 0; m < 3; ++m) b->conf[m] = batch_default_conf((dd_mode)m);
+  for (int m = 0; m < 3; ++m) b->conf[m] = batch_default_conf((dd_mode)m, false);
   *batch = b;
   return DD_OK;
 }
@@ -665,6 +684,7 @@ dd_status dd_batch_add_two_step(dd_batch *batch, dd_plan *plan, const uint8_t *d
 dd_status dd_batch_set_conf(dd_batch *batch, dd_mode mode, const dd_conf *conf) {
   if (!batch || !conf || (int)mode < 0 || (int)mode > 2) return fail(DD_ERR_INVALID_ARGUMENT, "invalid argument");
   batch->conf[mode] = *conf;
+  batch->conf_set[mode] = true;
   batch->invalidate();
   return DD_OK;
 }

@@ -455,6 +455,14 @@ void set_float_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, FloatKer
   g.lds_bytes = (uint32_t)lds_of(unroll, narrow);
 }
 
+// From the shapes of 128 sums per lane with 8 rows per barrier: 0.67 over 1536 rows and
+// 0.77 over 96 at 1.0 windows, 0.86 and 1.0 at 1.4 (it grows with the windows).
+float matrix_time_of(const dd_plan *p, dd_mode mode, const dd_conf &c) {
+  const uint32_t rows = mode == DD_SINGLE_STEP ? p->obs.nr_channels : cps(p);
+  const float windows = (mode == DD_SINGLE_STEP ? p->ish_single : p->ish_one).mean_windows(c.items_d1);
+  return (rows > 257 ? 0.67f : rows >= 64 ? 0.77f : 1.0f) * (0.3f + 0.7f * windows);
+}
+
 void set_byte_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, ByteKernel kernel, Geometry &g) {
   if (g.staged != 1 || mode == DD_STEP_TWO || p->input_bits == 32) return;
   const ShiftTable &t = mode == DD_SINGLE_STEP ? p->ish_single : p->ish_one;

@@ -165,6 +165,10 @@ enum class ByteKernel { kByRule, kVector, kMatrix };
 // matrix form has no such shape) and the LDS that it needs.
 void set_byte_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, ByteKernel kernel, Geometry &g);
 
+// The time of the matrix form of a byte launch in that of the vector form, in the
+// shapes that batches take.
+float matrix_time_of(const dd_plan *p, dd_mode mode, const dd_conf &c);
+
 // Which form of the staged float kernel a launch takes, likewise.
 enum class FloatKernel { kByRule, kOneCopy, kFourCopies };
 // Whether one copy of a row is faster under configuration c in a launch of `tiles` workgroups.
@@ -182,6 +186,7 @@ struct U8Launch {
   Geometry g{};
   dim3 grid;
   bool flush = false;
+  float matrix_time = 1.0f;  // matrix_time_of, in a batch
 };
 struct F32Launch {
   RowSumF32Params k{};

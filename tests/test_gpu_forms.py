@@ -124,6 +124,7 @@ SINGLE_BATCHES = [
     ("packed with bytes", [NARROW, dict(NARROW, bits=2, padding=0), dict(SEVERAL, bits=1), dict(NARROW, bits=4)], "matrix", True),
     ("mostly matrix", [dict(NARROW, samples=9000), SPREAD], "matrix", True),
     ("mostly vector", [NARROW, dict(SPREAD, samples=30000)], "staged", False),
+    ("half vector", [dict(NARROW, samples=3000, dms=64), dict(SPREAD, samples=3000, dms=64, step=2.0)], "staged", False),
     ("few rows", [FEW, FEW], "staged", False),
     ("one off a dword", [dict(NARROW, samples=9000), dict(NARROW, offset=1)], "staged", False),
     ("packed, one off a dword", [dict(NARROW, bits=2), dict(NARROW, bits=2, offset=3, samples=70)], "staged", False),
@@ -149,7 +150,7 @@ def test_single_step_batch(torch_cuda, case):
 
 @pytest.mark.parametrize("chunks", [0, 2])
 @pytest.mark.parametrize("compact", [True, False])
-@pytest.mark.parametrize("case", [c for c in SINGLE_BATCHES if c[0] not in ("few rows", "mostly vector")], ids=lambda c: c[0])
+@pytest.mark.parametrize("case", [c for c in SINGLE_BATCHES if c[0] not in ("few rows", "mostly vector", "half vector")], ids=lambda c: c[0])
 def test_two_step_batch(torch_cuda, case, compact, chunks):
     """Step one in the persistent launch and in the chunks' lists, as floats and as uint16 sums."""
     name, shapes, form, wide = case
@@ -429,3 +430,34 @@ def test_default_shape_of_wide_step_two(torch_cuda):
     plan = Plan(w.obs, 128)
     conf = plan.get_conf(DD_STEP_TWO)
     assert plan.launch_info(DD_STEP_TWO)["form"] == "groups" and (conf.threads_d1, conf.items_d0, conf.items_d1) == (8, 8, 4)
+
+
+# jobs (subbands, their step), the form of the batch that asks for the paired step two, its rows
+PAIRED = [
+    ("all pairs", [(16, 0.1), (6, 0.05)], "pairs", 8), ("one is odd", [(16, 0.1), (5, 0.05)], "pairs", 8),
+    ("many subbands", [(16, 0.1), (66, 0.05)], "pairs", 8),
+    ("one spreads too far", [(16, 0.1), (16, 1.0)], "whole", 4), ("one has no room", [(16, 1.0), (90, 0.05)], "staged", 4),
+]
+
+
+@pytest.mark.parametrize("chunks", [0, 2])
+@pytest.mark.parametrize("case", PAIRED, ids=lambda c: c[0])
+def test_paired_step_two_and_what_stands_in(torch_cuda, case, chunks):
+    """Where a job cannot take the paired step two, the batch runs what it would without asking."""
+    name, shapes, form, rows = case
+    jobs = [beam(s * 2, 900, 19, step, (1,), subbands=s, coarse=3, coarse_step=2.0, seed=80 + k)
+            for k, (s, step) in enumerate(shapes)]
+    forms = []
+    for paired in (False, True):
+        batch = Batch()
+        for j in jobs:
+            add(batch, j)
+            j["out"].fill_(-1.0)
+        batch.set_paired_step_two(paired)
+        batch.set_pipeline(chunks)
+        forms.append((batch.launch_info(DD_STEP_TWO)["form"], batch.get_conf(DD_STEP_TWO).unroll))
+        assert batch.info()["paired_step_two"] == (paired and form == "pairs")
+        batch.run(stream=stream_of(torch_cuda))
+        for k, j in enumerate(jobs):
+            verify(j, f"{name}, paired {paired}, chunks {chunks}, job {k}")
+    assert forms[1] == (form, rows) and (form == "pairs" or forms[0] == forms[1])
