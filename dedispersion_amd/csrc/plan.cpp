@@ -478,12 +478,14 @@ void set_byte_kernel(const dd_plan *p, dd_mode mode, const dd_conf &c, ByteKerne
       return 4 * (4 * slots + 3 * u * ((g.win + kU8MatrixReach) / 4) + 2 * (roundup(u, 4) + 4) * (tile + c.threads_d1)) + past;
     return 4 * (roundup(2 * slots, 4) + 2 * u * g.win + 2 * u * tile);
   };
+  // beside the matrix form's rows, the claim slot of a batch's kernel
+  auto limit = [&](bool matrix) { return p->max_lds - (matrix ? kClaimSlot : 0); };
   auto fitting = [&](bool matrix) {
     uint32_t u = std::min(c.unroll, kStagedSlotsPerWave * c.threads_d1);
-    while (u > 1 && lds_of(u, matrix) > p->max_lds) --u;
+    while (u > 1 && lds_of(u, matrix) > limit(matrix)) --u;
     return u;
   };
-  const bool shaped = (c.items_d1 == 4 || c.items_d1 == 8) && g.win <= kU8MatrixWindow && lds_of(1, true) <= p->max_lds;
+  const bool shaped = (c.items_d1 == 4 || c.items_d1 == 8) && g.win <= kU8MatrixWindow && lds_of(1, true) <= limit(true);
   g.matrix = shaped && (kernel == ByteKernel::kMatrix ||
                         (kernel == ByteKernel::kByRule && matrix_is_faster(slots, c, fitting(true), t)));
   // one window takes the first DM's shift modulo 8, the spread and the block's 8 samples

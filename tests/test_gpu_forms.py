@@ -461,3 +461,40 @@ def test_paired_step_two_and_what_stands_in(torch_cuda, case, chunks):
         for k, j in enumerate(jobs):
             verify(j, f"{name}, paired {paired}, chunks {chunks}, job {k}")
     assert forms[1] == (form, rows) and (form == "pairs" or forms[0] == forms[1])
+
+
+@pytest.mark.parametrize("two_step", [False, True])
+def test_matrix_batch_with_lds_to_the_last_byte(torch_cuda, two_step):
+    """A row list that fills LDS beside the rows per barrier: the persistent kernel's
+    claim slot has its room too, whatever the number of channels."""
+    mode = DD_STEP_ONE if two_step else DD_SINGLE_STEP
+    limit = 160 * 1024
+
+    def plan_of(channels):
+        w = workloads.tiny(channels=channels, samples=300, dms=1 if two_step else 8, step=0.01, min_freq=1250.0,
+                           bandwidth=300.0 / channels, coarse=8 if two_step else 0, coarse_step=0.01)
+        return Plan(w.obs, 128)
+
+    conf = Conf(64, 4, 16, 8, 8, 1)
+    base = plan_of(6000).launch_info(mode, conf)
+    assert base["form"] == "matrix" and base["rows_per_barrier"] == 8
+    channels = 6000 + (limit - base["lds_bytes"]) // 16  # 16 bytes per channel
+    rows = set()
+    for c in range(channels - 2, channels + 3):
+        plan = plan_of(c)
+        info = plan.launch_info(mode, conf)
+        assert info["form"] == "matrix" and info["lds_bytes"] <= limit - 16, (c, info)
+        rows.add(info["rows_per_barrier"])
+        z = plan.sizes
+        buffers = [torch_cuda.zeros(max(n, 1), dtype=d, device="cuda") for n, d in (
+            (max(z.input_elements, z.sub_input_elements), torch_cuda.uint8), (z.intermediate_elements, torch_cuda.float32),
+            (max(z.output_elements, z.sub_output_elements), torch_cuda.float32))]
+        batch = Batch()
+        if two_step:
+            batch.add_two_step(plan, *(b.data_ptr() for b in buffers))
+        else:
+            batch.add_single_step(plan, buffers[0].data_ptr(), buffers[2].data_ptr())
+        assert batch.launch_info(mode)["form"] == "matrix"
+        batch.run(stream=stream_of(torch_cuda))
+    assert rows == {7, 8}
+    torch_cuda.cuda.synchronize()
