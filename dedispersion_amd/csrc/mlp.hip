@@ -151,7 +151,9 @@ __device__ __forceinline__ void read_rows(const float *__restrict__ X, uint32_t 
         if (i + 4 <= inputs) {
           f = *reinterpret_cast<const Four *>(x);
         } else {
-          for (uint32_t k = 0; i + k < inputs; ++k) f.v[k] = x[k];
+#pragma unroll
+          for (uint32_t k = 0; k < 3; ++k)
+            if (i + k < inputs) f.v[k] = x[k];
         }
       }
 #pragma unroll
