@@ -561,10 +561,16 @@ dd_conf default_conf(const dd_plan *p, dd_mode mode) {
     // largest tile that still fills the device.  Measured over 420 plans of 1-64
     // subbands, 1-128 coarse and 1-96 fine DMs and 256-24576 samples, us in one group and
     // pipelined: 1 subband, 119 x 29 DMs x 7561 16.7 and 21.9; 8, 103 x 10 x 1093 6.0 and
-    // 9.0; 16, 50 x 10 x 2567 9.1 and 11.6; 32, 22 x 19 x 282 10.0 and 9.2.
-    if (o.nr_subbands <= 16) {
+    // 9.0; 16, 50 x 10 x 2567 9.1 and 11.6; 32, 22 x 19 x 282 10.0 and 9.2.  From 9
+    // subbands on, 33-40 DMs leave most of a second tile of 32 empty: in a grid that fills
+    // the device they take one pipelined tile of 64 (both steps, 16 subbands, 16 x 38 DMs x
+    // 13705 32.5 us, in groups 39.5).  Tiles of 16 DMs stay a little past the line where
+    // those of 32 fill the device (12 subbands, 23 x 21 DMs x 10063, 460 tiles of 32: 24.4
+    // and 29.8; 16 subbands, 10 x 78 x 4886, 300: 23.3 and 19.9).
+    const bool half_empty = o.nr_subbands > 8 && o.nr_dms > 32 && o.nr_dms <= 40 && tiles(32) >= cus;
+    if (o.nr_subbands <= 16 && !half_empty) {
       const uint32_t d1 = o.nr_dms <= 8 ? 1 : 2;
-      if (o.nr_dms > 16 && tiles(32) >= 2ull * cus) return conf_of(8, 8, 4, 8, 2);
+      if (o.nr_dms > 16 && 2 * tiles(32) >= 3ull * cus) return conf_of(8, 8, 4, 8, 2);
       return conf_of(8, 2 * tiles(8 * d1) >= cus ? 8 : 4, d1, 8, 2);
     }
     // Much output: small groups of rows and many workgroups per compute unit, once
