@@ -23,12 +23,12 @@
 //
 // Measured, 1459 rows, 2048 DMs x 24576 samples: 1.08 ms against 1.96 for the
 // vector form (68 T additions/s against 37); 1024 DMs x 12288 2-bit samples: 0.39
-// ms against 0.69.  Bounds: at two wavefronts per SIMD (128 sums per lane) a
-// product of 16 cycles takes 29, for the vector instructions that build the A
-// operands (a v_smfmac holds up its own wavefront's) and the LDS reads (half of
-// LDS's time); the 32x32x64 shape overlaps better but draws so much power that the
-// clock falls to 1.5 GHz (24 ns for the work that two of these do in 17).
-// Staging is a fifth of the time.
+// ms against 0.69.  Bounds, by the counters of the larger: the matrix cores are busy 43%
+// of the cycles, VALU issue 44% and LDS reads 60%, at two wavefronts per SIMD (128 sums
+// per lane).  A product of 16 cycles starts every 37, a fifth of which is staging; the
+// rest is the vector instructions that build the A operands (a v_smfmac holds up its
+// own wavefront's) and the reads.  The 32x32x64 shape overlaps better but draws so much
+// power that the clock falls to 1.5 GHz (24 ns for the work that two of these do in 17).
 #include "staged_common.hpp"
 #include "u8_unpack.hpp"
 
