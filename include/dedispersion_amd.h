@@ -72,7 +72,10 @@ typedef struct dd_observation {
  *   threads_d1  wavefronts along DMs per workgroup
  *   items_d0    samples per thread (4, 8 or 16)
  *   items_d1    DMs per thread (1, 2, 4 or 8)
- *   unroll      channels staged per barrier (1..16)
+ *   unroll      channels staged per barrier (1..16), at most: fewer where they
+ *               do not fit in LDS and, of float rows in grids of more
+ *               workgroups than compute units, where more workgroups then
+ *               share a unit (dd_plan_get_launch_info tells how many)
  *   local       0 = read rows through the caches; 1 = stage rows in LDS with
  *               a double-buffered pipeline (used when unroll <= 2 *
  *               threads_d1 and the row window fits, else as 2); 2 = stage
@@ -86,7 +89,13 @@ typedef struct dd_observation {
  *               blocks does not fit in LDS, run the staged pipeline.
  *               Local 1 and 2 whose row windows (the tile plus the spread
  *               of its DMs' shifts) do not fit in LDS run as local 0.
- *   split_batches must be 0 (unimplemented in the reference too). */
+ *               The pipeline of local 1 has more than one form (byte rows on
+ *               the matrix cores, float rows in four copies or one), chosen
+ *               by sizes; results do not depend on it.
+ *   split_batches must be 0 (unimplemented in the reference too).
+ * A plan starts with configurations chosen by its sizes, input type and
+ * shifts (dd_plan_get_conf); they are chosen again when one of these is set,
+ * until dd_plan_set_conf sets one. */
 typedef struct dd_conf {
   uint32_t threads_d0;
   uint32_t threads_d1;
@@ -402,7 +411,7 @@ dd_status dd_batch_set_compact_intermediate(dd_batch *batch, int enable);
  * difference takes at most 4 values per DM tile and the intermediate rows are
  * 8-element aligned; otherwise every subband is added on its own.  Results
  * are bit-identical either way.  On the 40-beam MI355X workload it is
- * slower than adding every subband (2.68 against 2.22 ms for the batch's step
+ * slower than adding every subband (2.68 against 1.98 ms for the batch's step
  * two), so it is an option.  No counterpart in the reference, whose step two
  * (include/Dedispersion.hpp:155-176) adds every subband. */
 dd_status dd_batch_set_paired_step_two(dd_batch *batch, int enable);
