@@ -246,8 +246,8 @@ dd_status plan_jobs(dd_batch *b, bool pairs, bool whole, ByteKernel single, Byte
         if (s == DD_ERR_CONFIGURATION) fits = false;
         else if (s != DD_OK) return s;
       } else if (fits) {
-        // one kernel for the batch: jobs whose row lists leave no room for one copy run beside it
-        fits = staged(L2) && (two != FloatKernel::kOneCopy || L2.g.narrow);
+        // one kernel for the batch: jobs whose rows do not fit in its form run beside it
+        fits = staged(L2) && (two == FloatKernel::kByRule || L2.g.narrow == (two == FloatKernel::kOneCopy));
       }
       b->beside.push_back(!fits);
       b->compact_job.push_back(fits && b->compact);
