@@ -75,12 +75,13 @@ struct ShiftTable {
   // per row and wavefront of `dms` consecutive DMs: the first DM's shift is
   // rounded down to 8 samples (3 on average) and an output block reaches 7
   // samples past the last DM's (cached per DM count like max_spread).  Taken over
-  // every fourth row: delays change little from one row to the next.
+  // every fourth row, and some 1024 of thousands: delays change little from one
+  // row to the next.
   float mean_windows(uint32_t dms) const {
     for (auto &c : window_cache)
       if (c.first == dms) return c.second;
     uint64_t sum = 0, n = 0;
-    for (uint32_t r = 0; r < rows; r += 4)
+    for (uint32_t r = 0; r < rows; r += std::max(rows / 1024, 4u))
       for (uint32_t d0 = 0; d0 < this->dms; d0 += dms, ++n)
         sum += 1 + (uint64_t)(at(r, std::min(d0 + dms - 1, pitch - 1)) - at(r, d0) + 10) / 32;
     const float mean = n ? (float)((double)sum / (double)n) : 1.0f;
